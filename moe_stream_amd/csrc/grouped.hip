@@ -41,7 +41,13 @@ __device__ __forceinline__ f32x4_t mfma16x16x32(uint4 a, uint4 b, f32x4_t c) {
 }
 
 constexpr int kTileM = 64;
-constexpr int kRsPitch = 80;   // row-sum LDS pitch (floats): 4 groups' rows on distinct banks
+// Wide items (twice the features) from this many of them on: four rounds of the
+// 512 resident workgroups.  Below it the last round and the longest items decide,
+// and narrow items are faster (512 tokens of Qwen3 1,256 wide down items; whole
+// block with the line at 512 / 1024 / 2048 wide items: gpt-oss 29 tokens 201 / 179
+// / 166 us, 256 tokens 469 / 470 / 449, Qwen3 256 tokens 126 / 122 / 116); past it
+// the wide item's halved token-row reads win.
+constexpr int kWideItems = 2048;
 
 // ---------------------------------------------------------------------------
 // grouping: one workgroup of 1024 threads; hist[] in dynamic LDS spans every
@@ -162,24 +168,27 @@ __global__ __launch_bounds__(1024) void group_pairs_kernel(
   group_pairs_body(refs, n_pairs, n_slots, n_records, D, perm, tiles, n_tiles, yp);
 }
 
-// B fragment: 8 codes of one weight row as bf16 128+q, x_pairs order.
-__device__ __forceinline__ uint4 b_frag(uint32_t w) {
-  uint32_t p[4];
-  codes_to_bf16x2(w, p);
-  return make_uint4(p[0], p[1], p[2], p[3]);
+// The fp32 sum of a row's group g as three bf16 parts whose sum is exact (3 x 8
+// significant bits): lane m < 3 of those that hold the sum writes part m.
+// row: [3][pitch], the pitch the groups rounded up to 32.
+__host__ __device__ constexpr int rs_pitch(int K) { return (K / 64 + 31) / 32 * 32; }
+__device__ __forceinline__ void put_row_sum(uint16_t *row, int pitch, int g, int m, float x) {
+  const float p0 = round_bf16(x), r = x - p0, p1 = round_bf16(r);
+  if (m < 3) row[m * pitch + g] = (uint16_t)f32_to_bf16(m == 0 ? p0 : m == 1 ? p1 : r - p1);
 }
 
 // ---------------------------------------------------------------------------
 // The A operand's rows in x_pairs order (each 8-input piece p holds inputs
 // (0,4), (1,5), (2,6), (3,7) pairwise, the order of the B fragments) and their
 // 64-input row sums, once per call: one thread per piece, the 8 pieces of a
-// group in 8 consecutive lanes (rs: [rows][K / 64] fp32).
+// group in 8 consecutive lanes (rs: [rows][3][rs_pitch(K)] bf16, see
+// put_row_sum).
 // ---------------------------------------------------------------------------
 // piece i of `rows` rows of K inputs (32-bit index arithmetic: the host
 // passes at most 2^30 pieces at a time)
 __device__ __forceinline__ void prep_piece(int i, const uint16_t *__restrict__ src, int64_t rows,
                                            int K, uint16_t *__restrict__ dst,
-                                           float *__restrict__ rs) {
+                                           uint16_t *__restrict__ rs) {
   const int ppr = K / 8;
   const bool ok = i < (int)(rows * ppr);
   const int r = ok ? i / ppr : 0;
@@ -195,14 +204,14 @@ __device__ __forceinline__ void prep_piece(int i, const uint16_t *__restrict__ s
   sm = group_sum<8>(sm);
   if (ok) {
     *reinterpret_cast<uint4 *>(dst + (int64_t)r * K + pc * 8) = make_uint4(out[0], out[1], out[2], out[3]);
-    if ((pc & 7) == 0) rs[(int64_t)r * (K / 64) + pc / 8] = sm;
+    put_row_sum(rs + (int64_t)r * (3 * rs_pitch(K)), rs_pitch(K), pc / 8, pc & 7, sm);
   }
 }
 
 __global__ __launch_bounds__(256) void grouped_prep_kernel(const uint16_t *__restrict__ src,
                                                            int64_t rows, int K,
                                                            uint16_t *__restrict__ dst,
-                                                           float *__restrict__ rs) {
+                                                           uint16_t *__restrict__ rs) {
   prep_piece(blockIdx.x * 256 + threadIdx.x, src, rows, K, dst, rs);
 }
 
@@ -212,7 +221,7 @@ __global__ __launch_bounds__(1024) void group_prep_kernel(
     const int32_t *__restrict__ refs, int n_pairs, int n_slots, int n_records, int D,
     int32_t *__restrict__ perm, int4 *__restrict__ tiles, int32_t *__restrict__ n_tiles,
     float *__restrict__ yp, const uint16_t *__restrict__ x, int64_t T, uint16_t *__restrict__ xq,
-    float *__restrict__ rsx) {
+    uint16_t *__restrict__ rsx) {
   if (blockIdx.x == 0)
     group_pairs_body(refs, n_pairs, n_slots, n_records, D, perm, tiles, n_tiles, yp);
   else
@@ -222,567 +231,630 @@ __global__ __launch_bounds__(1024) void group_prep_kernel(
 // ---------------------------------------------------------------------------
 // One work item of the grouped contraction: the rows of one tile (A, up to
 // 64 rows of KIN bf16 inputs, already in x_pairs order) against NPROJ
-// projections' 4-bit weights for NB consecutive output features.  WAVES
-// waves; wave w owns CPW 16-feature column blocks of every projection for
-// the NMB 16-row blocks the tile fills (a template parameter: no branches
-// around the MFMAs).
+// projections' 4-bit weights for 64 * CB consecutive output features, on 4
+// waves.  Wave w owns CB 16-feature column blocks of every projection for all
+// M 16-row blocks the tile fills (a template parameter: no branches around
+// the MFMAs).
 //
-// The inputs are processed a quad (4 quant groups of 64 inputs) at a time.
-// A quad's operands sit in LDS while the workgroup computes its 4 groups
-// with no barrier in between; the next quad's operands wait in registers
-// (their loads issued a quad earlier) and go to LDS between two barriers at
-// the quad's end, when the loads of the quad after it are issued.
-//  * A: the token rows' 8-input pieces, row-major per group, piece p of row r
-//    at r * 8 + (p ^ (r & 7)): each 8-lane run of the copy writes one whole
-//    row (no bank conflict) and the MFMA reads of a piece across 16 rows fall
-//    on distinct banks.
-//  * B: 128 bytes of every weight row per quad (whole cache lines, 8 lanes
-//    per row); in LDS 8 chunks of 16 bytes, chunk c at c ^ ((row >> 1) & 7),
-//    so the 32 lanes of one 8-byte fragment read (16 rows x 2 halves) fall on
-//    distinct banks.  Each lane reads its two code words (8 bytes) per group.
-// Every thread issues the same loads on every path (rows past the tile and
-// chunks past the row are clamped to a valid address and never used; the
-// last quads are unrolled), so the compiler's counter waits ask for exactly
-// the data in hand.  The item's scales, biases and row sums are staged in
-// LDS once: scales quad-major (each lane reads its row's 4 scales of a quad
-// as 8 contiguous bytes, the 16 rows of a fragment side by side), row sums at
-// a pitch of 80 floats (the 4 groups of one bias MFMA on distinct banks).
-// Each group accumulates into a fresh 16x16 block (2 MFMAs over the bf16
-// 128+q codes), folded into the output by S; the bias term
-// sum_g rowsum[g] * (B - 128 S) runs on fp32 MFMAs (K = 4 groups) per quad.
+//  * A: one quad (4 quant groups of 64 inputs) of the tile's rows in LDS, in
+//    two buffers, one barrier per quad: while a quad is computed the next
+//    one's pieces are loaded into registers half a quad at a time and written
+//    to the other buffer.  Piece p of row r of a group sits at
+//    r * 8 + (p ^ (r & 7)): the 8 lanes that copy a row and the 16 rows of a
+//    fragment read both fall on distinct banks.
+//  * B: each wave loads its own rows' codes (64 bytes of a row by 4 lanes) a
+//    quad ahead into registers and turns them into fragments through an LDS
+//    region of its own, half a quad at a time and without a barrier: chunk c of
+//    row r at c ^ (r >> 2), so the 32 lanes of an 8-byte fragment read fall on
+//    distinct banks.  (Loaded in fragment order, 16 rows per 16 lanes, each
+//    8-byte piece costs a cache access of its own.)
+//  * Each group accumulates into a fresh 16x16 block (2 MFMAs over the bf16
+//    128+q codes), folded into the output by S.
+//  * The scale rows sit in LDS for the whole item (read 8 bytes at a time from
+//    memory they cost a cache line per row and quad).
+//  * The bias term sum_g rowsum[g] * (B[g] - 128 S[g]) starts the output
+//    block: three bf16 MFMAs of the row sums' parts against the B row and three
+//    against the S row (the record's own bf16 values) give it with exact
+//    products and fp32 sums.
+//
+// Measured (whole block against the previous kernels: 64-row tiles with codes and
+// rows staged a quad at a time behind two barriers, the bias term on fp32 MFMAs;
+// cold weights): Qwen3 4,096 tokens 698 -> 585 us, gpt-oss 700 tokens 747 -> 640,
+// gpt-oss 29 tokens 210 -> 166.  A full gate/up tile now spends 30 of its 44 us in
+// the quads, two waves per SIMD at about half the MFMA rate; the rest is the first
+// operands' latency and the epilogue.  One-block tiles are bound by HBM and that
+// latency.
+//
+// What sets the shape: per group a wave's M x N blocks (N = CB * NPROJ) take
+// 32 M N matrix-core cycles, 64 M LDS cycles (a 16-row fragment is 2 KB, the
+// CU's LDS serves four SIMDs at 128 B/cycle) and 4 * (14 N + 4 M N) VALU cycles
+// (decode of 2 N code words, fold).  At M = 4 the LDS reads alone exceed the
+// MFMAs for N < 2; at N = 4 they are half of them and the VALU work is level.
 // Rows past the tile compute garbage from a copy of a real row, which no
-// output row depends on (MFMA rows are independent) and nothing stores.
+// output row depends on (MFMA rows are independent) and nothing stores;
+// features past the matrix likewise (their addresses are clamped).
 // ---------------------------------------------------------------------------
-template <int KIN, int NB, int WAVES, int NPROJ>
-struct GItem {
-  static constexpr int NT = 64 * WAVES;
-  static constexpr int NG = KIN / 64;                  // quant groups along the inputs
-  static constexpr int NQ = (NG + 3) / 4;              // quads (B staging units)
-  static constexpr int NG4 = NQ;                       // bias MFMAs, 4 groups each
-  static constexpr int CPW = NB / 16 / WAVES;          // column blocks per wave
-  static constexpr int SPT = (kTileM * 8 + NT - 1) / NT;   // A pieces per thread and group
-  static constexpr int BROWS = NPROJ * NB;             // weight rows of the item
-  static constexpr int BPT = BROWS * 8 / NT;           // B 16-byte pieces per thread and quad
-  static constexpr int SCB = NB * NG * 2;              // bytes of one scale array's block
-  static constexpr int NARR = 2 * NPROJ;               // (S, B) per projection
-  static constexpr int SCP = NARR * SCB / 16;          // 16-byte pieces of all of them
-  static constexpr int SCW = (SCP + NT - 1) / NT;      // ... per thread
-  // with NG a multiple of 4 the scales are staged quad-major: [array][quad][feature]
-  // x 4 halfwords (8-byte pieces), else copied as they are ([array][feature][group])
-  static constexpr bool QS = NG % 4 == 0;
-  static constexpr int SQP = NARR * NQ * NB;           // 8-byte pieces, quad-major
-  static constexpr int SQW = (SQP + NT - 1) / NT;      // ... per thread
-  static constexpr int RSW = (NG4 * 4 + WAVES - 1) / WAVES;   // row-sum groups per thread
-  static_assert(KIN % 64 == 0 && NB % (16 * WAVES) == 0 && CPW >= 1, "feature split");
-  static_assert(SCB % 16 == 0 && NT % 8 == 0 && (BROWS * 8) % NT == 0, "staging");
-  // quads [0, QMAIN) refill the registers with quad q + 2 (a loop); the last
-  // two quads are unrolled
-  static constexpr int QMAIN = NQ >= 2 ? NQ - 2 : 0;
+constexpr int kCodeBytes = 4096;   // a wave's code region: 4 blocks of 16 rows x 64 bytes
+
+template <int KIN>
+struct GDim {
+  static constexpr int NG = KIN / 64;             // quant groups along the inputs
+  static constexpr int NQ = (NG + 3) / 4;         // quads
+  static constexpr int NGL = NG - 4 * (NQ - 1);   // groups of the last quad
+  // scale rows in LDS: as they are where a quad's 4 halfwords are then 8-byte
+  // aligned, else each padded to 16 bytes
+  static constexpr bool SRAW = NG % 4 == 0;
+  static constexpr int SPB = SRAW ? NG * 2 : (NG + 7) / 8 * 16;   // row pitch, bytes
+  static constexpr int SPP = SPB;                 // 16-byte pieces of a block's 16 rows
+  static constexpr int KS = (NG + 31) / 32;       // bias MFMA steps (32 groups each)
+  static_assert(KIN % 64 == 0, "whole quant groups");
 };
 
-struct GLds {   // (one layout for every instantiation; sized by the caller)
-  float *part;             // gate/up with the fused input prep: [NB / 16][64] row partial sums
-  int *rperm;              // down: the tile rows' pair ids [64] ...
-  float *rsc;              // ... and their scores [64]
-  uint4 (*a)[kTileM * 8];  // [4 groups][row * 8 + (piece ^ (row & 7))]
-  uint4 *b;                // [BROWS][8]: one quad of codes
-  float *rs;               // [NG4 * 4][kRsPitch]: 64-input row sums (row < 64), zero past NG
-  uint4 *sc;
+constexpr int kMmWaves = 4, kMmThreads = 64 * kMmWaves;
+
+typedef u32x4_t u32x4_a4_t __attribute__((aligned(4)));
+__device__ __forceinline__ uint32_t gload2(const void *p) {
+  return *(const __attribute__((address_space(1))) uint16_t *)(p);
+}
+
+// keeps halfwords [0, v) of a 16-byte fragment
+__device__ __forceinline__ uint4 keep_halves(uint4 f, int v) {
+  auto m = [&](int w) { return 2 * w + 1 < v ? 0xffffffffu : 2 * w < v ? 0xffffu : 0u; };
+  return make_uint4(f.x & m(0), f.y & m(1), f.z & m(2), f.w & m(3));
+}
+
+// Chunk ci of a row of NG (odd or small) bf16 values, 2-byte aligned: halfwords
+// 8 ci .. + 7, zero past NG.  The load never leaves the row's dwords (a window
+// across the row's end is read 8 halfwords before it and shifted) and is
+// dword-aligned: a 16-byte load at an odd halfword takes several times as long.
+template <int NG>
+__device__ __forceinline__ uint4 row_chunk(const char *row, int ci) {
+  if (NG < 8) {
+    uint32_t h[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) h[i] = i < NG ? gload2(row + 2 * (i < NG ? i : 0)) : 0u;
+    return make_uint4(h[0] | (h[1] << 16), h[2] | (h[3] << 16), h[4] | (h[5] << 16),
+                      h[6] | (h[7] << 16));
+  }
+  constexpr int SH = 8 - NG % 8;   // of the window across the end
+  const int b = 8 * ci;
+  const char *p = row + min(b, NG - 8) * 2;
+  const uint32_t odd = (uint32_t)(uintptr_t)p & 2u;
+  const char *p4 = p - odd;
+  const u32x4_t f = *(const __attribute__((address_space(1))) u32x4_a4_t *)(p4);
+  const uint32_t l = (uint32_t)gload4i(p4 + (odd ? 16 : 12));
+  const uint32_t x[5] = {f.x, f.y, f.z, f.w, l};
+  uint32_t w[8] = {0, 0, 0, 0, 0, 0, 0, 0}, t[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) w[i] = odd ? (x[i] >> 16) | (x[i + 1] << 16) : x[i];
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+    t[i] = SH % 2 ? (w[i + SH / 2] >> 16) | (w[i + SH / 2 + 1] << 16) : w[i + SH / 2];
+  return b > NG - 8 ? make_uint4(t[0], t[1], t[2], t[3]) : make_uint4(w[0], w[1], w[2], w[3]);
+}
+
+// Fragment of 8 halfwords of a scale row in LDS (8-byte aligned)
+__device__ __forceinline__ uint4 lds_frag(const char *p, int v) {
+  const uint2 a = reinterpret_cast<const uint2 *>(p)[0], b = reinterpret_cast<const uint2 *>(p)[1];
+  return keep_halves(make_uint4(a.x, a.y, b.x, b.y), v);
+}
+
+// sigmoid in fp32, about 2 ulp: exp(-x) as exp2 of the product's leading part
+// with its remainder applied to first order, and one Newton step on the
+// reciprocal (of expf and the division it takes a third of the instructions;
+// the activation is a fifth of a full tile's VALU work).  Past +-87 it is 1 or
+// 2^-126 to within fp32's range.
+__device__ __forceinline__ float sigmoid_f32(float x) {
+  x = fminf(fmaxf(x, -87.f), 87.f);
+  const float hi = x * -1.44269502f;                        // -log2(e), leading part
+  const float lo = fmaf(x, -1.44269502f, -hi) + x * -1.92596303e-8f;
+  float e = __builtin_amdgcn_exp2f(hi);
+  e = fmaf(e, lo * 0.693147181f, e);
+  const float d = 1.f + e, r = __builtin_amdgcn_rcpf(d);
+  return fmaf(fmaf(-d, r, 1.f), r, r);
+}
+__device__ __forceinline__ float gated_act(int act, float g, float u, float alpha, float limit) {
+  if (act == MOE_ACT_SWIGLU) return g * sigmoid_f32(g) * u;
+  g = fminf(g, limit);
+  u = fminf(fmaxf(u, -limit), limit);
+  return g * sigmoid_f32(alpha * g) * (u + 1.f);
+}
+
+struct GLds {
+  uint4 *a;                    // two buffers of [groups][row * 8 + (piece ^ (row & 7))]
+  char *b;                     // [4 waves][N blocks][16 rows][64 bytes], swizzled
+  char *s;                     // [4 waves][N blocks][16 rows][SPB bytes]: the scales
+  int *rperm;                  // down: the tile rows' pair ids [64] ...
+  float *rsc;                  // ... and their scores [64]
 };
 
-template <int NMB, int D, int F, bool PBIAS, int NB, int WAVES, bool GU>
+// pair / k by the multiplier ceil(2^32 / k), exact for pairs below 2^24 and
+// k <= 32; k == 1 has no such multiplier and takes the pair itself (no branch:
+// the rows' loads hang on this)
+struct TokenOf {
+  uint32_t mul, one;
+  __device__ __forceinline__ int operator()(int pair) const {
+    return (int)(__umulhi((uint32_t)pair, mul) + ((uint32_t)pair & one));
+  }
+};
+static TokenOf token_of(int k) {
+  if (k == 1) return {0u, ~0u};
+  return {(uint32_t)((((uint64_t)1 << 32) + k - 1) / k), 0u};
+}
+
+// Keeps the value's computation here in program order (emits nothing).
+template <class T>
+__device__ __forceinline__ void pin(T &v) {
+  asm volatile("" : "+v"(v));
+}
+
+template <int M, int CB, int D, int F, bool PBIAS, bool GU>
 __device__ __forceinline__ void grouped_item(
-    const PoolArgs &pa, const uint16_t *__restrict__ aq, const float *__restrict__ ars, int k,
-    const int32_t *__restrict__ perm, int ref, int r0, int rows, int nb0,
-    uint16_t *__restrict__ h_out, float *__restrict__ rs_out, const float *__restrict__ scores,
-    float *__restrict__ yp, int act, float alpha, float limit, const GLds &L) {
-  constexpr int KIN = GU ? D : F, NPROJ = GU ? 2 : 1;
-  using I = GItem<KIN, NB, WAVES, NPROJ>;
-  constexpr int NG = I::NG, NQ = I::NQ, CPW = I::CPW, NT = I::NT, SPT = I::SPT;
-  constexpr int BPT = I::BPT;
-  constexpr int NP = PBIAS ? 4 : 3, SCH = I::SCB / 2;   // halfwords per scale array block
-  constexpr int ROWS = NMB * 16;                        // staged rows
-  constexpr int RB = KIN / 2;                           // bytes per weight row
-  const uint16_t *sch = reinterpret_cast<const uint16_t *>(L.sc);
+    const PoolArgs &pa, const uint16_t *__restrict__ aq, const uint16_t *__restrict__ ars,
+    TokenOf tok, const int32_t *__restrict__ perm, int ref, int r0, int rows, int nb0,
+    uint16_t *__restrict__ h_out, uint16_t *__restrict__ rs_out,
+    const float *__restrict__ scores, float *__restrict__ yp, int act, float alpha, float limit,
+    const GLds &L) {
+  constexpr int KIN = GU ? D : F, NOUT = GU ? F : D, NPROJ = GU ? 2 : 1;
+  using I = GDim<KIN>;
+  constexpr int NG = I::NG, NQ = I::NQ, NGL = I::NGL, KS = I::KS, SPB = I::SPB;
+  constexpr int NP = PBIAS ? 4 : 3, NB = 16 * CB * kMmWaves, RB = KIN / 2;
+  constexpr int ROWS = 16 * M;
+  // A in LDS: whole quads of 32 rows, or half quads of 64; R quads wait in
+  // registers
+  constexpr bool QA = M <= 2;
+  constexpr int AROWS = QA ? 32 : 64, AG = QA ? 4 : 2, R = M == 1 ? 2 : 1;
+  constexpr int SPG = AROWS * 8 / kMmThreads;   // A pieces per thread and group
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int col = lane & 15, kq = lane >> 4;
-  const char *w[NPROJ];
-  const char *sa[I::NARR];
+  // (named, not arrays: a pointer picked from an array by a lane's index goes
+  // through memory)
+  constexpr int PF = GU ? PROJ_GATE : PROJ_DOWN, PL = GU ? PROJ_UP : PROJ_DOWN;
+  const char *const w0 = resolve(pa, comp_index(PF, PART_W, NP), ref);
+  const char *const w1 = resolve(pa, comp_index(PL, PART_W, NP), ref);
+  const char *const s0 = resolve(pa, comp_index(PF, PART_S, NP), ref);
+  const char *const s1 = resolve(pa, comp_index(PL, PART_S, NP), ref);
+  const char *const o0 = resolve(pa, comp_index(PF, PART_B, NP), ref);
+  const char *const o1 = resolve(pa, comp_index(PL, PART_B, NP), ref);
+  constexpr int N = CB * NPROJ;                        // blocks of a wave
+  constexpr int NG0 = NQ > 1 ? 4 : NGL;                // groups of the first quad
+  // the row indices first: everything else of the tile's rows hangs on them
+  auto row_index = [&](int r) { return gload4i(perm + r0 + min(r, rows - 1)); };
+  int pr_st[SPG], pr_rs = 0, pr_ep = 0;
 #pragma unroll
-  for (int j = 0; j < NPROJ; ++j) {
-    const int proj = GU ? (j == 0 ? PROJ_GATE : PROJ_UP) : PROJ_DOWN;
-    w[j] = resolve(pa, comp_index(proj, PART_W, NP), ref);
-    sa[2 * j] = resolve(pa, comp_index(proj, PART_S, NP), ref);
-    sa[2 * j + 1] = resolve(pa, comp_index(proj, PART_B, NP), ref);
-  }
-  // the A source row of tile row r (clamped into the tile)
-  auto src_row = [&](int r) -> int64_t {
-    r = min(r, rows - 1);
-    return GU ? gload4i(perm + r0 + r) / k : r0 + r;
+  for (int j = 0; j < SPG; ++j) pr_st[j] = GU ? row_index((tid >> 3) + 32 * j) : 0;
+  if (GU) pr_rs = row_index(tid >> 2);
+  if (!GU) pr_ep = row_index(lane);
+  // codes of half a quad: lane l of a wave loads 16-byte chunk l & 3 of row l >>
+  // 2 of each of its blocks
+  uint32_t boff[CB];
+  const int bch = (lane & 3) * 16;
+#pragma unroll
+  for (int cb = 0; cb < CB; ++cb)
+    boff[cb] = (uint32_t)min(nb0 + (wave * CB + cb) * 16 + (lane >> 2), NOUT - 1) * RB;
+  uint4 breg[R][2][N];   // codes to come
+  auto load_b = [&](int q, int hf, int rs) {
+    // (chunks past the row, in a last partial quad: its last one, unused)
+    const int o = q * 128 + hf * 64;
+    const uint32_t c = RB % 64 == 0 || o + 64 <= RB ? (uint32_t)(o + bch)
+                                                    : (uint32_t)min(o + bch, RB - 16);
+#pragma unroll
+    for (int n = 0; n < N; ++n) 
+      breg[rs][hf][n] = gload16((n % NPROJ ? w1 : w0) + boff[n / NPROJ] + c);
   };
-  // this thread's A pieces (slot s = 8 * row + piece)
-  const uint16_t *asrc[SPT];
+  char *const bl = L.b + wave * kCodeBytes;
+  const uint32_t bwr = (uint32_t)((lane >> 2) * 64 + (((lane & 3) ^ (lane >> 4)) << 4));
+  // (a wave's own region: its LDS accesses are in order, the fences keep the
+  // compiler from moving one lane's reads across another's writes)
+  auto store_b = [&](int hf, int rs) {
+    asm volatile("" ::: "memory");
 #pragma unroll
-  for (int j = 0; j < SPT; ++j) {
-    const int s = tid + NT * j;
-    asrc[j] = aq + src_row(s >> 3) * KIN + (s & 7) * 8;
-  }
-  auto load_a = [&](int g, uint4 (&v)[SPT]) {
-#pragma unroll
-    for (int j = 0; j < SPT; ++j) v[j] = gload16(asrc[j] + g * 64);
+    for (int n = 0; n < N; ++n) *reinterpret_cast<uint4 *>(bl + n * 1024 + bwr) = breg[rs][hf][n];
+    asm volatile("" ::: "memory");
   };
-  // this thread's B pieces: piece p = tid + NT * i is chunk p % 8 of item
-  // weight row p / 8 (rows [0, NB) the first projection, then the second)
-  const char *bsrc[BPT];
-  uint32_t bdst[BPT];   // LDS byte offset of the piece in the quad buffer
+  // this lane's 16 codes of a group: row col of block n, bytes 8 kq .. + 7
+  const uint32_t brd = (uint32_t)(col * 64 + (((kq >> 1) ^ (col >> 2)) << 4) + (kq & 1) * 8);
+  auto read_b = [&](int gi, int n) {
+    return *reinterpret_cast<const uint2 *>(bl + n * 1024 + (brd ^ ((gi & 1) << 5)));
+  };
+  // the wave's scale rows (and, for the bias term, bias rows), all of the
+  // item, as SPP 16-byte pieces per block of 16 rows (contiguous memory where
+  // the rows stay as they are, else a chunk of a row); a pass takes PB blocks (as
+  // many as fit the code region, which the bias rows pass through), lane l its
+  // pieces l, l + 64, ...
+  constexpr int SPP = I::SPP, PB = N * 16 * SPB <= kCodeBytes ? N : N / 2, NPASS = N / PB;
+  constexpr int NPC = PB * SPP, PT = (NPC + 63) / 64;
+  static_assert(PB >= 1 && PB * 16 * SPB <= kCodeBytes && N % PB == 0, "bias rows in the code region");
+  char *const sl = L.s + wave * (N * 16 * SPB);
+  auto scale_piece = [&](int h, int t, const char *a0, const char *a1) {
+    const int i = min(lane + 64 * t, NPC - 1), n = h * PB + i / SPP, o = i % SPP;
+    const int f = min(nb0 + (wave * CB + n / NPROJ) * 16, NOUT - 16);
+    const char *p = (NPROJ > 1 && (n & 1) ? a1 : a0) + (uint32_t)(f * (NG * 2));
+    if (I::SRAW) return gload16(p + o * 16);
+    return row_chunk<NG>(p + o / (SPB / 16) * (NG * 2), o % (SPB / 16));
+  };
+  auto store_piece = [&](char *dst, int t, uint4 v) {   // into a pass's rows
+    const int i = lane + 64 * t;
+    if (NPC % 64 == 0 || i < NPC) *reinterpret_cast<uint4 *>(dst + i * 16) = v;
+  };
+  // A: this thread's pieces of the rows (tid >> 3) + 32 j, half a quad at a time
+  const uint16_t *asrc[SPG];
+  uint32_t adst[SPG];
+  uint4 areg[R][AG][SPG];
+  // groups g0 .. g0 + AG - 1 of a quad, as many as its ng
+  auto load_a = [&](int q, int g0, int ng, int rs) {
 #pragma unroll
-  for (int i = 0; i < BPT; ++i) {
-    const int p = tid + NT * i, row = p >> 3, c = p & 7;
-    const int j = row / NB, fl = row % NB;
-    bsrc[i] = w[NPROJ > 1 ? j : 0] + (int64_t)(nb0 + fl) * RB + c * 16;
-    bdst[i] = (uint32_t)(row * 128 + ((c ^ ((row >> 1) & 7)) << 4));
-  }
-  auto load_b = [&](int q, uint4 (&v)[BPT]) {
+    for (int i = 0; i < AG; ++i)
+      if (g0 + i < ng)
 #pragma unroll
-    for (int i = 0; i < BPT; ++i) {
-      // (a chunk past the row end, in a last partial quad: any valid chunk)
-      const int off = (RB % 128 == 0 || q * 128 + 128 <= RB)
-                          ? q * 128
-                          : min(q * 128, RB - 16 - (int)((tid + NT * i) & 7) * 16);
-      v[i] = gload16(bsrc[i] + off);
+        for (int j = 0; j < SPG; ++j) areg[rs][i][j] = gload16(asrc[j] + (q * 4 + g0 + i) * 64);
+  };
+  auto store_a = [&](int buf, int g0, int ng, int rs) {
+#pragma unroll
+    for (int i = 0; i < AG; ++i)
+      if (g0 + i < ng)
+#pragma unroll
+        for (int j = 0; j < SPG; ++j)
+          L.a[(buf * AG + i) * (AROWS * 8) + adst[j]] = areg[rs][i][j];
+  };
+  // the scales, the first codes, the row sums' parts and the first A rows on
+  // their way
+  uint4 sv[NPASS][PT], bv[NPASS][PT];
+#pragma unroll
+  for (int h = 0; h < NPASS; ++h)
+#pragma unroll
+    for (int t = 0; t < PT; ++t) {
+      sv[h][t] = scale_piece(h, t, s0, s1);
+      bv[h][t] = scale_piece(h, t, o0, o1);
     }
-  };
-  auto store_b = [&](int buf, const uint4 (&v)[BPT]) {
-    char *base = reinterpret_cast<char *>(L.b + buf * I::BROWS * 8);
-#pragma unroll
-    for (int i = 0; i < BPT; ++i) *reinterpret_cast<uint4 *>(base + bdst[i]) = v[i];
-  };
-  // this lane's B fragment rows: feature col of column block cb, projection j
-  uint32_t bfr[NPROJ][CPW];   // LDS byte offset of the row in a quad buffer
-  uint32_t bx[NPROJ][CPW];    // its chunk swizzle ((row >> 1) & 7), as a byte offset
+  float pb[NPROJ][CB];
 #pragma unroll
   for (int j = 0; j < NPROJ; ++j)
 #pragma unroll
-    for (int cb = 0; cb < CPW; ++cb) {
-      const int row = j * NB + (wave * CPW + cb) * 16 + col;
-      bfr[j][cb] = row * 128;
-      bx[j][cb] = ((row >> 1) & 7) << 4;
-    }
-  // the item's scales and biases (each array's NB rows are one contiguous
-  // block) and row sums, loaded ahead of the first quad and written to LDS after
-  constexpr bool QS = I::QS;
-  constexpr int SCN = QS ? I::SQW : I::SCW;
-  uint4 scv[QS ? 1 : I::SCW];
-  uint2 sqv[QS ? I::SQW : 1];
-#pragma unroll
-  for (int j = 0; j < SCN; ++j) {
-    if (QS) {   // piece i: feature i % NB, quad (i / NB) % NQ, array i / (NB * NQ)
-      const int i = min(tid + NT * j, I::SQP - 1);
-      const int nl = i % NB, q = (i / NB) % NQ, arr = i / (NB * NQ);
-      sqv[j] = gload8(sa[arr] + ((int64_t)(nb0 + nl) * NG + 4 * q) * 2);
-    } else {
-      const int i = min(tid + NT * j, I::SCP - 1);
-      const int arr = i / (I::SCB / 16), o = i % (I::SCB / 16);
-      scv[j] = gload16(sa[arr] + (int64_t)nb0 * NG * 2 + (int64_t)o * 16);
-    }
-  }
-  float rsv[I::RSW];
-  {
-    const float *rrow = ars + src_row(lane) * NG;
-#pragma unroll
-    for (int j = 0; j < I::RSW; ++j) rsv[j] = gload4f(rrow + min(wave + WAVES * j, NG - 1));
-  }
-  // one quad of token-row pieces and codes in registers at a time
-  uint4 breg[BPT];
-  uint4 areg[4][SPT];
-  auto load_quad = [&](int q, int ng) {   // ng: the quad's groups (a constant)
-#pragma unroll
-    for (int gi = 0; gi < 4; ++gi)
-      if (gi < ng) load_a(4 * q + gi, areg[gi]);
-    load_b(q, breg);
-  };
-  auto store_quad = [&](int ng) {
-#pragma unroll
-    for (int gi = 0; gi < 4; ++gi) {
-      if (gi >= ng) continue;
-#pragma unroll
-      for (int j = 0; j < SPT; ++j) {
-        const int sl = tid + NT * j;
-        if (sl < ROWS * 8) {   // uniform per wave
-          const int r = sl >> 3, p = sl & 7;
-          L.a[gi][r * 8 + (p ^ (r & 7))] = areg[gi][j];
-        }
-      }
-    }
-    store_b(0, breg);
-  };
-  constexpr int NGL = NG - 4 * (NQ - 1);   // groups of the last quad
-  load_quad(0, NQ > 1 ? 4 : NGL);
-  // down: the pair id and score of tile row `lane` for the epilogue (every
-  // wave loads them, wave 0 keeps them: no branch around the loads)
-  int my_pr = 0;
-  float my_sc = 0.f;
-  if (!GU) {
-    my_pr = gload4i(perm + r0 + min(lane, rows - 1));
-    my_sc = gload4f(scores + my_pr);
-  }
-#pragma unroll
-  for (int j = 0; j < SCN; ++j) {
-    if (QS) {
-      if (I::SQP % NT == 0 || tid + NT * j < I::SQP)
-        reinterpret_cast<uint2 *>(L.sc)[tid + NT * j] = sqv[j];
-    } else {
-      if (I::SCP % NT == 0 || tid + NT * j < I::SCP) L.sc[tid + NT * j] = scv[j];
-    }
-  }
-#pragma unroll
-  for (int j = 0; j < I::RSW; ++j) {
-    const int g = wave + WAVES * j;
-    if (g < I::NG4 * 4) L.rs[g * kRsPitch + lane] = g < NG ? rsv[j] : 0.f;
-  }
-  f32x4_t acc[NMB][CPW][NPROJ];
-#pragma unroll
-  for (int rb = 0; rb < NMB; ++rb)
-#pragma unroll
-    for (int cb = 0; cb < CPW; ++cb)
-#pragma unroll
-      for (int j = 0; j < NPROJ; ++j) acc[rb][cb][j] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
-  store_quad(NQ > 1 ? 4 : NGL);
-  if (!GU && wave == 0) {
-    L.rperm[lane] = my_pr;
-    L.rsc[lane] = my_sc;
-  }
-  if (NQ > 1) load_quad(1, NQ > 2 ? 4 : NGL);
-  __syncthreads();
-  // with quad-major scales each lane reads its row's scales 4 groups at a
-  // time (8 bytes at the quad's first group)
-  const uint2 *scq = reinterpret_cast<const uint2 *>(L.sc);
-  uint2 s4[NPROJ][CPW];
-  // the bias term of quad q: fp32 MFMAs of K = 4 groups, A = row sums (lane:
-  // row col, group 4q + kq), B = B - 128 S of this lane's feature (zero past
-  // NG).  Each starts from a zero accumulator and is added on the VALU (no
-  // MFMA reads registers as its accumulator input: see below).
-  auto bias_step = [&](int q, const uint2 (&s4)[NPROJ][CPW]) {
-    const int gb = 4 * q + kq, gc = min(gb, NG - 1);
-    float C[NPROJ][CPW];
-#pragma unroll
-    for (int j = 0; j < NPROJ; ++j)
-#pragma unroll
-      for (int cb = 0; cb < CPW; ++cb) {
-        const int nl = (wave * CPW + cb) * 16 + col;
-        float sv, bv;
-        if (QS) {   // this lane's group of the quad from the quad's 4 halfwords
-          const uint2 b4 = scq[((2 * j + 1) * NQ + q) * NB + nl];
-          const uint32_t hs = kq < 2 ? s4[j][cb].x : s4[j][cb].y;
-          const uint32_t hb = kq < 2 ? b4.x : b4.y;
-          sv = __uint_as_float((kq & 1) ? (hs & 0xffff0000u) : (hs << 16));
-          bv = __uint_as_float((kq & 1) ? (hb & 0xffff0000u) : (hb << 16));
-        } else {
-          sv = bf16_to_f32(sch[(2 * j) * SCH + nl * NG + gc]);
-          bv = bf16_to_f32(sch[(2 * j + 1) * SCH + nl * NG + gc]);
-        }
-        C[j][cb] = gb < NG ? bv - 128.f * sv : 0.f;
-      }
-#pragma unroll
-    for (int rb = 0; rb < NMB; ++rb) {
-      const float ra = L.rs[gb * kRsPitch + rb * 16 + col];
-#pragma unroll
-      for (int cb = 0; cb < CPW; ++cb)
-#pragma unroll
-        for (int j = 0; j < NPROJ; ++j) {
-          const f32x4_t bz = __builtin_amdgcn_mfma_f32_16x16x4f32(
-              ra, C[j][cb], (f32x4_t){0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
-#pragma unroll
-          for (int e = 0; e < 4; ++e) acc[rb][cb][j][e] += bz[e];
-        }
-    }
-  };
-  // One group of the quad in LDS (gi: its index in the quad, a constant), in
-  // source order: decode, MFMAs, fold (down, held to 128 VGPRs)
-  auto group = [&](int g, int gi) {
-    if (QS && gi == 0) {   // the quad's scales, 4 halfwords per lane and row
-#pragma unroll
-      for (int j = 0; j < NPROJ; ++j)
-#pragma unroll
-        for (int cb = 0; cb < CPW; ++cb) {
-          const int nl = (wave * CPW + cb) * 16 + col;
-          s4[j][cb] = scq[((2 * j) * NQ + (g >> 2)) * NB + nl];
-        }
-    }
-    const uint4 *al = L.a[gi];
-    const char *bq = reinterpret_cast<const char *>(L.b);
-    const uint32_t cpos = (uint32_t)(gi * 32 + kq * 8);   // logical chunk and half
-    uint4 b0[NPROJ][CPW], b1[NPROJ][CPW];
-    float S[NPROJ][CPW];
-#pragma unroll
-    for (int j = 0; j < NPROJ; ++j)
-#pragma unroll
-      for (int cb = 0; cb < CPW; ++cb) {
-        const uint2 cw = *reinterpret_cast<const uint2 *>(bq + bfr[j][cb] + (cpos ^ bx[j][cb]));
-        b0[j][cb] = b_frag(cw.x);
-        b1[j][cb] = b_frag(cw.y);
-        if (QS) {
-          const uint32_t h = gi < 2 ? s4[j][cb].x : s4[j][cb].y;
-          S[j][cb] = __uint_as_float((gi & 1) ? (h & 0xffff0000u) : (h << 16));
-        } else {
-          const int nl = (wave * CPW + cb) * 16 + col;
-          S[j][cb] = bf16_to_f32(sch[(2 * j) * SCH + nl * NG + g]);
-        }
-      }
-#pragma unroll
-    for (int rb = 0; rb < NMB; ++rb) {
-      const int r = rb * 16 + col;
-      const uint4 a0 = al[r * 8 + ((2 * kq) ^ (r & 7))], a1 = al[r * 8 + ((2 * kq + 1) ^ (r & 7))];
-#pragma unroll
-      for (int cb = 0; cb < CPW; ++cb)
-#pragma unroll
-        for (int j = 0; j < NPROJ; ++j) {
-          const f32x4_t c0 = mfma16x16x32(a0, b0[j][cb], (f32x4_t){0.f, 0.f, 0.f, 0.f});
-          const f32x4_t c = mfma16x16x32(a1, b1[j][cb], c0);
-#pragma unroll
-          for (int e = 0; e < 4; ++e) acc[rb][cb][j][e] += S[j][cb] * c[e];
-          // c0 (the second MFMA's accumulator input) stays allocated until the
-          // fold has read c: this compiler otherwise reuses its registers a
-          // few instructions after the MFMA issues, before the MFMA has read
-          // them.  The empty asm passes acc through (a data dependency, not a
-          // side effect), so it orders no memory access and LDS reads of
-          // later row blocks can still be issued ahead of this fold
-          asm("" : "+v"(acc[rb][cb][j]) : "v"(c0));
-        }
-    }
-  };
-  // One group of the quad in LDS (gi: its index in the quad, a constant), in
-  // three steps so the quad can run them as a software pipeline: its B
-  // fragments decoded (and its scales), its MFMAs into fresh 16x16 blocks, and
-  // the fold of those blocks into the output by S.  The quad issues group
-  // gi's MFMAs, then decodes group gi + 1 and folds group gi, so that VALU
-  // work independent of the MFMAs in flight follows them.
-  struct GFrag {
-    uint4 b0[NPROJ][CPW], b1[NPROJ][CPW];
-    float S[NPROJ][CPW];
-  };
-  struct GOut {
-    f32x4_t c0[NMB][CPW][NPROJ], c[NMB][CPW][NPROJ];
-  };
-  auto decode = [&](int g, int gi, GFrag &f) {
-    if (QS && gi == 0) {   // the quad's scales, 4 halfwords per lane and row
-#pragma unroll
-      for (int j = 0; j < NPROJ; ++j)
-#pragma unroll
-        for (int cb = 0; cb < CPW; ++cb) {
-          const int nl = (wave * CPW + cb) * 16 + col;
-          s4[j][cb] = scq[((2 * j) * NQ + (g >> 2)) * NB + nl];
-        }
-    }
-    const char *bq = reinterpret_cast<const char *>(L.b);
-    const uint32_t cpos = (uint32_t)(gi * 32 + kq * 8);   // logical chunk and half
-#pragma unroll
-    for (int j = 0; j < NPROJ; ++j)
-#pragma unroll
-      for (int cb = 0; cb < CPW; ++cb) {
-        const uint2 cw = *reinterpret_cast<const uint2 *>(bq + bfr[j][cb] + (cpos ^ bx[j][cb]));
-        f.b0[j][cb] = b_frag(cw.x);
-        f.b1[j][cb] = b_frag(cw.y);
-        if (QS) {
-          const uint32_t h = gi < 2 ? s4[j][cb].x : s4[j][cb].y;
-          f.S[j][cb] = __uint_as_float((gi & 1) ? (h & 0xffff0000u) : (h << 16));
-        } else {
-          const int nl = (wave * CPW + cb) * 16 + col;
-          f.S[j][cb] = bf16_to_f32(sch[(2 * j) * SCH + nl * NG + g]);
-        }
-      }
-  };
-  auto mma = [&](int gi, const GFrag &f, GOut &o) {
-    const uint4 *al = L.a[gi];
-#pragma unroll
-    for (int rb = 0; rb < NMB; ++rb) {
-      const int r = rb * 16 + col;
-      const uint4 a0 = al[r * 8 + ((2 * kq) ^ (r & 7))], a1 = al[r * 8 + ((2 * kq + 1) ^ (r & 7))];
-#pragma unroll
-      for (int cb = 0; cb < CPW; ++cb)
-#pragma unroll
-        for (int j = 0; j < NPROJ; ++j) {
-          o.c0[rb][cb][j] = mfma16x16x32(a0, f.b0[j][cb], (f32x4_t){0.f, 0.f, 0.f, 0.f});
-          o.c[rb][cb][j] = mfma16x16x32(a1, f.b1[j][cb], o.c0[rb][cb][j]);
-        }
-    }
-  };
-  auto fold = [&](const GFrag &f, const GOut &o) {
-#pragma unroll
-    for (int rb = 0; rb < NMB; ++rb)
-#pragma unroll
-      for (int cb = 0; cb < CPW; ++cb)
-#pragma unroll
-        for (int j = 0; j < NPROJ; ++j) {
-#pragma unroll
-          for (int e = 0; e < 4; ++e) acc[rb][cb][j][e] += f.S[j][cb] * o.c[rb][cb][j][e];
-          // c0 (the second MFMA's accumulator input) stays allocated until the
-          // fold has read c: this compiler otherwise reuses its registers a
-          // few instructions after the MFMA issues, before the MFMA has read
-          // them.  The empty asm passes acc through (a data dependency, not a
-          // side effect), so it orders no memory access
-          asm("" : "+v"(acc[rb][cb][j]) : "v"(o.c0[rb][cb][j]));
-        }
-  };
-  // one quad: its groups from LDS, its bias term; then (all waves done with
-  // the quad) the next quad's operands from registers to LDS and the loads of
-  // the one after
-  auto quad = [&](int q, int ng, bool next, int ng_next, bool refill, int ng_refill) {
-    if (GU && QS) {   // gate/up: the pipelined order (down keeps 4 waves per
-                      // SIMD; with NG % 4 != 0 it would not fit 256 VGPRs)
-      GFrag fr[2];
-      GOut o;
-      decode(4 * q, 0, fr[0]);
-#pragma unroll
-      for (int gi = 0; gi < 4; ++gi) {
-        if (gi >= ng) continue;
-        mma(gi, fr[gi & 1], o);
-        if (gi + 1 < ng) decode(4 * q + gi + 1, gi + 1, fr[(gi + 1) & 1]);
-        fold(fr[gi & 1], o);
-      }
-    } else {
-#pragma unroll
-      for (int gi = 0; gi < 4; ++gi)
-        if (gi < ng) group(4 * q + gi, gi);
-    }
-    bias_step(q, s4);
-    if (next) {
-      __syncthreads();
-      store_quad(ng_next);
-      if (refill) load_quad(q + 2, ng_refill);
-      __syncthreads();
-    }
-  };
-  for (int q = 0; q < I::QMAIN; ++q) quad(q, 4, true, 4, true, q + 2 < NQ - 1 ? 4 : NGL);
-  if (NQ >= 2) quad(NQ - 2, 4, true, NGL, false, 0);
-  quad(NQ - 1, NGL, false, 0, false, 0);
-  // epilogue.  The item's output tile goes through LDS (the quad buffers,
-  // free once every wave is past the last quad) and out as whole rows, 16
-  // bytes per lane.  Gate/up with NB a multiple of 64 also does the down
-  // kernel's input prep: h goes out in x_pairs order (feature f of an
-  // 8-feature piece at 2 * (f % 4) + f / 4) with the sums of its bf16 values
-  // over each 64-feature group (16 features per 16-lane row, then 4 column
-  // blocks in order through LDS).  Down scales each row by its score.
-  constexpr bool FUSE = GU && NB % 64 == 0;
-  constexpr int OB = GU ? 2 : 4;                          // output bytes per element
-  constexpr bool STAGE = ROWS * NB * OB <= (int)(4 * kTileM * 8 * sizeof(uint4));
-  // the staged tile's element swizzle: XOR with 16 x ((row >> 2) & mask), the
-  // mask kept so that an element never leaves its row (NB features)
-  constexpr int SWM = NB % 64 == 0 ? 3 : NB % 32 == 0 ? 1 : 0;
-  auto swz = [](int r) { return ((r >> 2) & SWM) << 4; };
-  __syncthreads();
-  char *tile = reinterpret_cast<char *>(L.a[0]);
-#pragma unroll
-  for (int cb = 0; cb < CPW; ++cb) {
-    const int nl = (wave * CPW + cb) * 16 + col, n = nb0 + nl;
-    const int npl = FUSE ? (nl & ~7) + ((nl & 3) << 1) + ((nl >> 2) & 1) : nl;
-    float pb[NPROJ];
-#pragma unroll
-    for (int j = 0; j < NPROJ; ++j) {
-      pb[j] = 0.f;
+    for (int cb = 0; cb < CB; ++cb) {
+      pb[j][cb] = 0.f;
       if (PBIAS) {
         const int proj = GU ? (j == 0 ? PROJ_GATE : PROJ_UP) : PROJ_DOWN;
-        pb[j] = bf16_to_f32(reinterpret_cast<const uint16_t *>(
-            resolve(pa, comp_index(proj, PART_BIAS, NP), ref))[n]);
+        const int f = min(nb0 + (wave * CB + cb) * 16 + col, NOUT - 1);
+        pb[j][cb] =
+            bf16_to_f32(gload2(resolve(pa, comp_index(proj, PART_BIAS, NP), ref) + 2 * f));
       }
     }
+  load_b(0, 0, 0);
+  if (NG0 > 2) load_b(0, 1, 0);
+  constexpr int NGP = rs_pitch(KIN), RSP = 6 * NGP + 16, RSJ = 6 * NGP / 64;
+  static_assert(64 * RSP <= 4 * kTileM * 8 * 16, "row-sum parts in the A buffers");
+  uint4 rsv[RSJ];
+  {
+    const int64_t row = GU ? tok(pr_rs) : r0 + min(tid >> 2, rows - 1);
+    const char *src = reinterpret_cast<const char *>(ars + row * (3 * NGP)) + (tid & 3) * 16;
 #pragma unroll
-    for (int rb = 0; rb < NMB; ++rb) {
+    for (int i = 0; i < RSJ; ++i) rsv[i] = gload16(src + 64 * i);
+  }
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int rr = rb * 16 + 4 * kq + e;   // (uniform over each 16-lane row)
-        // staged tile: row rr, element npl ^ swz(rr) (the 4 rows of one
-        // store fall on distinct banks)
-        const int ec = npl ^ swz(rr);
-        if (GU) {
-          const float hv = apply_act(act, acc[rb][cb][0][e] + pb[0],
-                                     acc[rb][cb][NPROJ - 1][e] + pb[NPROJ - 1], alpha, limit);
-          const uint32_t hb = f32_to_bf16(hv);
-          if (STAGE)
-            reinterpret_cast<uint16_t *>(tile)[rr * NB + ec] = (uint16_t)hb;
-          else if (rr < rows)
-            h_out[(int64_t)(r0 + rr) * F + nb0 + npl] = (uint16_t)hb;
-          if (FUSE) {
-            const float ps = group_sum<16>(bf16_to_f32(hb));
-            if (col == 0) L.part[(wave * CPW + cb) * kTileM + rr] = ps;
+  for (int j = 0; j < SPG; ++j) {
+    const int r = (tid >> 3) + 32 * j, p = tid & 7;
+    const int64_t arow = GU ? tok(pr_st[j]) : r0 + min(r, rows - 1);
+    asrc[j] = aq + arow * KIN + p * 8;
+    adst[j] = (uint32_t)(r * 8 + (p ^ (r & 7)));
+  }
+  load_a(0, 0, NG0, 0);
+  f32x4_t acc[M][CB][NPROJ];
+#pragma unroll
+  for (int rb = 0; rb < M; ++rb)
+#pragma unroll
+    for (int cb = 0; cb < CB; ++cb)
+#pragma unroll
+      for (int j = 0; j < NPROJ; ++j) acc[rb][cb][j] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+  if (!GU && wave == 0) {
+    L.rperm[lane] = pr_ep;
+    L.rsc[lane] = gload4f(scores + pr_ep);
+  }
+#pragma unroll
+  for (int h = 0; h < NPASS; ++h)
+#pragma unroll
+    for (int t = 0; t < PT; ++t) store_piece(sl + h * (PB * 16 * SPB), t, sv[h][t]);
+  {
+    char *const rl = reinterpret_cast<char *>(L.a) + (tid >> 2) * RSP + (tid & 3) * 16;
+#pragma unroll
+    for (int i = 0; i < RSJ; ++i) *reinterpret_cast<uint4 *>(rl + 64 * i) = rsv[i];
+  }
+  __syncthreads();
+  // the output blocks start from the bias term
+#pragma unroll
+  for (int h = 0; h < NPASS; ++h) {
+    asm volatile("" ::: "memory");
+#pragma unroll
+    for (int t = 0; t < PT; ++t) store_piece(bl, t, bv[h][t]);
+    asm volatile("" ::: "memory");
+#pragma unroll
+    for (int i = 0; i < PB; ++i) {
+      const int n = h * PB + i, cb = n / NPROJ, j = n % NPROJ;
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) {
+        // (chunks past the row: any, all zeroed)
+        const int ci = min(4 * ks + kq, (NG - 1) / 8), v = max(0, min(8, NG - (32 * ks + 8 * kq)));
+        const uint4 fs = lds_frag(sl + (n * 16 + col) * SPB + ci * 16, v);
+        const uint4 fb = lds_frag(bl + (i * 16 + col) * SPB + ci * 16, v);
+#pragma unroll
+        for (int rb = 0; rb < M; ++rb) {
+          const char *ra = reinterpret_cast<const char *>(L.a) + (rb * 16 + col) * RSP + ks * 64 + kq * 16;
+          f32x4_t cs = {0.f, 0.f, 0.f, 0.f};
+          f32x4_t &o = acc[rb][cb][j];
+#pragma unroll
+          for (int p = 0; p < 3; ++p) {
+            uint4 a = *reinterpret_cast<const uint4 *>(ra + p * 2 * NGP);
+            if (NG % 32) a = keep_halves(a, v);
+            o = mfma16x16x32(a, fb, o);
+            cs = mfma16x16x32(a, fs, cs);
           }
-        } else {
-          const float v = acc[rb][cb][0][e] + pb[0];
-          if (STAGE) {
-            reinterpret_cast<float *>(tile)[rr * NB + ec] = L.rsc[rr] * v;
-          } else if (rr < rows) {
-            const int pr = L.rperm[rr];
-            yp[(int64_t)pr * D + n] = L.rsc[rr] * v;
-          }
+#pragma unroll
+          for (int e = 0; e < 4; ++e) o[e] -= 128.f * cs[e];
         }
       }
     }
   }
+  __syncthreads();   // the row-sum parts are read
+  store_a(0, 0, NG0, 0);
+  store_b(0, 0);
+  // quads 1 .. R on their way (of the A rows whole quads only)
+#pragma unroll
+  for (int q = 1; q <= R; ++q)
+    if (q < NQ) {
+      if (QA) load_a(q, 0, q < NQ - 1 ? 4 : NGL, q % R);
+      load_b(q, 0, q % R);
+      if (R > 1 && q < R) load_b(q, 1, q % R);
+    }
   __syncthreads();
-  if (STAGE) {   // whole rows out, 16 bytes per lane
-    constexpr int CPR = NB * OB / 16;                     // 16-byte chunks per row
-    constexpr int EPC = 16 / OB;                          // elements per chunk
-    // (the thread index made opaque: the LDS addresses below are computed
-    // here, not held in registers across the work items)
-    int tid_e = tid;
-    asm volatile("" : "+v"(tid_e));
-#pragma unroll 1
-    for (int it = 0; it < (ROWS * CPR + NT - 1) / NT; ++it) {
-      const int i = tid_e + NT * it, r = i / CPR, c = i % CPR;
-      if (i < ROWS * CPR && r < rows) {
-        const int ec = (c * EPC) ^ swz(r);
-        const uint4 v = *reinterpret_cast<const uint4 *>(tile + (r * NB + ec) * OB);
-        if (GU)
-          *reinterpret_cast<uint4 *>(h_out + (int64_t)(r0 + r) * F + nb0 + c * EPC) = v;
-        else
-          *reinterpret_cast<uint4 *>(yp + (int64_t)L.rperm[r] * D + nb0 + c * EPC) = v;
+  // The quads as a software pipeline of steps, one per (group, block n of the
+  // wave's N): a step issues its 2 M MFMAs into fresh blocks, and between them
+  // the VALU work of its neighbours: ahead of each first MFMA the fold of the
+  // step before out of the block it overwrites (4 instructions, that MFMA's own
+  // 16 cycles), behind the second ones the decode of the step after.  The order
+  // is pinned: left to itself the compiler puts each fold right behind its
+  // MFMAs and waits for them.
+  uint4 a0[M], a1[M];     // the group's A fragments (inputs 0-31 and 32-63 of the lane order)
+  uint32_t bf[2][8];      // a step's B fragments: both halves
+  uint2 creg[2];          // codes of the steps after
+  f32x4_t c[M];           // its blocks
+  float S[2];
+  uint2 scur[N];          // the quad's scales
+  int ard[2];             // LDS index of this lane's two pieces in row block 0
+  ard[0] = col * 8 + ((2 * kq) ^ (col & 7));
+  ard[1] = col * 8 + ((2 * kq + 1) ^ (col & 7));
+#pragma unroll
+  for (int rb = 0; rb < M; ++rb) {
+    a0[rb] = L.a[rb * 128 + ard[0]];
+    a1[rb] = L.a[rb * 128 + ard[1]];
+    c[rb] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+  }
+  S[1] = 0.f;
+#pragma unroll
+  for (int n = 0; n < N; ++n)
+    scur[n] = *reinterpret_cast<const uint2 *>(sl + (n * 16 + col) * SPB);
+  // fragment word m of 8, 4 of each code word, as pairs of bf16 128+q (one
+  // v_and_or_b32 after the shift: its constants in registers.  Not bfi_mask():
+  // the compiler does not see that an inline instruction writes a register
+  // that an MFMA in flight still reads)
+  uint32_t kmask = 0x000f000fu, kexp = 0x43004300u;
+  pin(kmask);
+  pin(kexp);
+  auto decode = [&](uint2 cw, int m) {
+    return (((m < 4 ? cw.x : cw.y) >> (4 * (m & 3))) & kmask) | kexp;
+  };
+  creg[0] = read_b(0, 0);
+  creg[1] = read_b(1 / N, 1 % N);
+#pragma unroll
+  for (int m = 0; m < 8; ++m) bf[0][m] = decode(creg[0], m);
+  // One quad of ng groups (constants, as is everything but q; par: its parity):
+  // steps s = gi * N + n, the step registers alternating by s.  Two steps
+  // before the end of each half, when the last of its codes are read, the next
+  // half's go from registers to the wave's own LDS and the loads of the same
+  // half R quads on are issued into the registers (ng_next, ng_second, ng_load:
+  // groups of quads q + 1, q + R and q + 1 + R, 0: none).  The A rows of the
+  // next quad go along with M <= 2, else half a quad ahead.  The barrier is one
+  // step before the quad's (half's) end, so that the last step can read the
+  // next fragments.
+  auto quad = [&](int q, int par, int ng, int ng_next, int ng_second, int ng_load) {
+    const int ns = ng * N, rs = (par + 1) % R;
+#pragma unroll
+    for (int st = 0; st < 4 * N; ++st) {
+      if (st >= ns) continue;
+      const int gi = st / N, n = st % N, j = n % NPROJ, cb = n / NPROJ;
+      const int cur = st & 1, prv = cur ^ 1;
+      // the block folded here: the step before's
+      const int pn = (n + N - 1) % N, pj = pn % NPROJ, pcb = pn / NPROJ;
+      const bool dec = st + 1 < ns || ng_next > 0;   // there is a step after
+      const bool last = st + 1 == ns;
+      const bool half_end = last || (!QA && st == 2 * N - 1);
+      const int nbuf = QA ? par ^ 1 : last ? 0 : 1;   // the A buffer after this one
+      if (!QA && st == 0 && ng > 2) load_a(q, 2, ng, 0);
+      if (!QA && st == (ng > 2 ? 2 * N : 0) && ng_next > 0) load_a(q + 1, 0, ng_next, 0);
+      if (!QA && half_end && (!last || ng_next > 0))
+        store_a(nbuf, last ? 0 : 2, last ? ng_next : ng, 0);
+      // codes: the second half's when the last of the first are read ...
+      if (ng > 2 && st + 2 == 2 * N) {
+        store_b(1, par % R);
+        if (ng_second > 2) load_b(q + R, 1, par % R);
+      }
+      // ... and the next quad's
+      if (st + 2 == ns && ng_next > 0) {
+        if (QA) store_a(par ^ 1, 0, ng_next, rs);
+        store_b(0, rs);
+        if (ng_load > 0) {
+          if (QA) load_a(q + 1 + R, 0, ng_load, rs);
+          load_b(q + 1 + R, 0, rs);
+        }
+      }
+      if (half_end && (!last || ng_next > 0)) __syncthreads();
+      // codes of the step after next
+      if (st + 2 < ns)
+        creg[cur] = read_b((st + 2) / N, (st + 2) % N);
+      else if (ng_next > 0)
+        creg[cur] = read_b((st + 2 - ns) / N, (st + 2 - ns) % N);
+      // A fragments of the next group, on a group's last step
+      const bool nxa = n == N - 1 && dec;
+      const int ag = half_end ? nbuf * AG : QA ? par * AG + gi + 1 : gi + 1;
+      const uint4 *an = L.a + ag * (AROWS * 8);
+      const uint32_t h = gi < 2 ? scur[n].x : scur[n].y;
+      S[cur] = __uint_as_float((gi & 1) ? (h & 0xffff0000u) : (h << 16));
+      if (last && ng_next > 0)
+#pragma unroll
+        for (int i = 0; i < N; ++i)
+          scur[i] = *reinterpret_cast<const uint2 *>(sl + (i * 16 + col) * SPB + (q + 1) * 8);
+      const uint4 fb0 = make_uint4(bf[cur][0], bf[cur][1], bf[cur][2], bf[cur][3]);
+      const uint4 fb1 = make_uint4(bf[cur][4], bf[cur][5], bf[cur][6], bf[cur][7]);
+      uint2 cw = creg[prv];
+      if (dec) pin(cw.x), pin(cw.y);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int rb = 0; rb < M; ++rb) {
+        f32x4_t &o = acc[rb][pcb][pj];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) o[e] += S[prv] * c[rb][e];
+        pin(o);
+        c[rb] = mfma16x16x32(a0[rb], fb0, (f32x4_t){0.f, 0.f, 0.f, 0.f});
+        pin(c[rb]);
+        if (nxa) a0[rb] = an[rb * 128 + ard[0]];
+        __builtin_amdgcn_sched_barrier(0);
+      }
+#pragma unroll
+      for (int rb = 0; rb < M; ++rb) {
+        c[rb] = mfma16x16x32(a1[rb], fb1, c[rb]);
+        pin(c[rb]);
+        if (nxa) a1[rb] = an[rb * 128 + ard[1]];
+        if (dec)
+#pragma unroll
+          for (int m = 8 * rb / M; m < 8 * (rb + 1) / M; ++m)
+            bf[prv][m] = decode(cw, m), pin(bf[prv][m]);
+        __builtin_amdgcn_sched_barrier(0);
       }
     }
+  };
+  // the quads whose loads are whole quads (in pairs where the registers
+  // alternate), then the rest
+  constexpr int QR = R == 2 || QA ? 2 : 1, QP = NQ > R + 2 ? (NQ - R - 2) / QR * QR : 0;
+#pragma unroll 1
+  for (int q = 0; q < QP; q += QR) {
+    quad(q, 0, 4, 4, 4, 4);
+    if (QR == 2) quad(q + 1, 1, 4, 4, 4, 4);
   }
-  if (FUSE) {
 #pragma unroll
-    for (int i = tid; i < ROWS * (NB / 64); i += NT) {
-      const int r = i % ROWS, gq = i / ROWS;
-      if (r < rows) {
-        float sm = 0.f;
+  for (int q = QP; q < NQ; ++q) {
+    auto groups = [](int i) { return i < NQ - 1 ? 4 : i == NQ - 1 ? NGL : 0; };
+    quad(q, q & 1, groups(q), groups(q + 1), groups(q + R), groups(q + 1 + R));
+  }
+  {   // the last step's fold
+    constexpr int last = (NGL * N - 1) & 1;
 #pragma unroll
-        for (int c = 0; c < 4; ++c) sm += L.part[(gq * 4 + c) * kTileM + r];
-        rs_out[(int64_t)(r0 + r) * (F / 64) + nb0 / 64 + gq] = sm;
+    for (int rb = 0; rb < M; ++rb)
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        acc[rb][(N - 1) / NPROJ][(N - 1) % NPROJ][e] += S[last] * c[rb][e];
+  }
+
+  if (GU) {
+    // the activations go through LDS (the A buffers, free once every wave is
+    // past the last quad) and out as whole rows, 16 bytes per lane, in x_pairs
+    // order (feature f of an 8-feature piece at 2 * (f % 4) + f / 4) with the
+    // sums of their bf16 values over each 64-feature group, the down kernel's
+    // input.  Staged element npl of row r at npl ^ 16 * ((r >> 2) & 3) (the 4
+    // rows of one store fall on distinct banks).
+    static_assert(NB % 64 == 0 && F % 64 == 0, "whole groups of h");
+    __syncthreads();
+    uint16_t *tile = reinterpret_cast<uint16_t *>(L.a);
+    auto swz = [](int r) { return ((r >> 2) & 3) << 4; };
+#pragma unroll
+    for (int cb = 0; cb < CB; ++cb) {
+      const int nl = (wave * CB + cb) * 16 + col;
+      const int npl = (nl & ~7) + ((nl & 3) << 1) + ((nl >> 2) & 1);
+#pragma unroll
+      for (int rb = 0; rb < M; ++rb)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int rr = rb * 16 + 4 * kq + e;
+          const float hv = gated_act(act, acc[rb][cb][0][e] + pb[0][cb],
+                                     acc[rb][cb][NPROJ - 1][e] + pb[NPROJ - 1][cb], alpha, limit);
+          tile[rr * NB + (npl ^ swz(rr))] = (uint16_t)f32_to_bf16(hv);
+        }
+    }
+    __syncthreads();
+    constexpr int CPR = NB / 8;                       // 16-byte pieces per row
+#pragma unroll 1
+    for (int i = tid; i < ROWS * CPR; i += kMmThreads) {
+      const int r = i / CPR, c = i % CPR, f = nb0 + c * 8;
+      const uint4 v = *reinterpret_cast<const uint4 *>(tile + r * NB + ((c * 8) ^ swz(r)));
+      const uint32_t in[4] = {v.x, v.y, v.z, v.w};
+      float sm = 0.f;
+#pragma unroll
+      for (int m = 0; m < 4; ++m) sm += bf16_to_f32(in[m] & 0xffffu) + bf16_to_f32(in[m] >> 16);
+      sm = group_sum<8>(sm);
+      if (r < rows && f < F) {
+        *reinterpret_cast<uint4 *>(h_out + (int64_t)(r0 + r) * F + f) = v;
+        put_row_sum(rs_out + (int64_t)(r0 + r) * (3 * rs_pitch(F)), rs_pitch(F), f / 64, c & 7, sm);
+      }
+    }
+  } else {
+    // each row scaled by its score, through LDS (the A buffers) and out as whole
+    // rows, 16 bytes per lane, 32 rows at a time.  Staged element nl of row r at
+    // nl ^ 16 * ((r >> 2) & 3).
+    float *tile = reinterpret_cast<float *>(L.a);
+    constexpr int CPR = NB / 4;   // 16-byte pieces per row
+    static_assert(32 * NB * 4 <= 4 * kTileM * 8 * 16, "32 rows in the A buffers");
+#pragma unroll
+    for (int r2 = 0; r2 < M; r2 += 2) {
+      __syncthreads();
+#pragma unroll
+      for (int rb = r2; rb < (r2 + 2 < M ? r2 + 2 : M); ++rb)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int rr = rb * 16 + 4 * kq + e;
+          const float sc = L.rsc[rr];
+#pragma unroll
+          for (int cb = 0; cb < CB; ++cb)
+            tile[(rr - r2 * 16) * NB + (((wave * CB + cb) * 16 + col) ^ (kq << 4))] =
+                sc * (acc[rb][cb][0][e] + pb[0][cb]);
+        }
+      __syncthreads();
+#pragma unroll 4
+      for (int i = tid; i < 32 * CPR; i += kMmThreads) {
+        const int r = i / CPR, cc = (i % CPR) * 4, rr = r2 * 16 + r;
+        if (rr < rows && (D % NB == 0 || nb0 + cc < D))
+          *reinterpret_cast<uint4 *>(yp + (int64_t)L.rperm[rr] * D + nb0 + cc) =
+              *reinterpret_cast<const uint4 *>(tile + r * NB + (cc ^ (((r >> 2) & 3) << 4)));
       }
     }
   }
 }
 
-template <int D, int F, bool PBIAS, int NB, int WAVES, bool GU>
-__global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(WAVES == 8 && !GU ? 4 : 2))) void grouped_mm_kernel(
-    PoolArgs pa, const uint16_t *__restrict__ aq, const float *__restrict__ ars, int k,
-    const int32_t *__restrict__ perm, const int4 *__restrict__ tiles,
-    const int32_t *__restrict__ n_tiles, uint16_t *__restrict__ h_out,
-    float *__restrict__ rs_out, const float *__restrict__ scores, float *__restrict__ yp,
-    int act, float alpha,
-    float limit) {
-  constexpr int KIN = GU ? D : F, NOUT = GU ? F : D, NPROJ = GU ? 2 : 1;
-  constexpr int NBK = NOUT / NB, NP = PBIAS ? 4 : 3;
-  using I = GItem<KIN, NB, WAVES, NPROJ>;
-  static_assert(NOUT % NB == 0, "whole feature blocks");
-  __shared__ uint4 a_l[4][kTileM * 8];
-  __shared__ uint4 b_l[I::BROWS * 8];
-  __shared__ float rs_l[I::NG4 * 4 * kRsPitch];
-  __shared__ uint4 sc_l[I::QS ? (I::SQP + 1) / 2 : I::SCP];
-  __shared__ float pt_l[GU && NB % 64 == 0 ? NB / 16 * kTileM : 1];
-  __shared__ int rp_l[GU ? 1 : kTileM];
-  __shared__ float rc_l[GU ? 1 : kTileM];
-  const GLds L{pt_l, rp_l, rc_l, a_l, b_l, rs_l, sc_l};
-  const int n_items = *n_tiles * NBK;
+// Items of a call: (tile, feature block).  From kXcdTiles tiles on the items
+// of one tile go to workgroups of one XCD (workgroup i runs on XCD i % 8), so
+// the tile's rows are read from HBM once and from that XCD's L2 by the other
+// items, and a hot expert's codes once per XCD.  With fewer tiles that would
+// leave XCDs idle; the items are dealt in order.
+constexpr int kXcdTiles = 64;
+
+template <int CB, int D, int F, bool PBIAS, bool GU>
+__device__ __forceinline__ void grouped_items(
+    const PoolArgs &pa, const uint16_t *aq, const uint16_t *ars, TokenOf tok,
+    const int32_t *perm, const int4 *tiles, int n_tiles, uint16_t *h_out, uint16_t *rs_out,
+    const float *scores, float *yp, int act, float alpha, float limit, const GLds &L) {
+  constexpr int NOUT = GU ? F : D, NB = 16 * CB * kMmWaves, NBK = (NOUT + NB - 1) / NB;
+  constexpr int NP = PBIAS ? 4 : 3, NPROJ = GU ? 2 : 1;
+  const bool by_xcd = n_tiles >= kXcdTiles;
+  const int n_items = (by_xcd ? (n_tiles + 7) / 8 * 8 : n_tiles) * NBK;
   for (int item = blockIdx.x; item < n_items; item += gridDim.x) {
-    const int4 tl = tiles[item / NBK];
+    const int j = item >> 3;
+    const int tile = by_xcd ? (j / NBK) * 8 + (item & 7) : item / NBK;
+    const int nb0 = (by_xcd ? j % NBK : item % NBK) * NB;
+    if (tile >= n_tiles) continue;
+    const int4 tl = tiles[tile];
     const int ref = tl.x, r0 = tl.y, rows = tl.z;
-    const int nb0 = (item % NBK) * NB;
     bool bad = false;
 #pragma unroll
-    for (int j = 0; j < NPROJ; ++j) {
-      const int proj = GU ? (j == 0 ? PROJ_GATE : PROJ_UP) : PROJ_DOWN;
+    for (int p = 0; p < NPROJ; ++p) {
+      const int proj = GU ? (p == 0 ? PROJ_GATE : PROJ_UP) : PROJ_DOWN;
       bad = bad || resolve(pa, comp_index(proj, PART_W, NP), ref) == nullptr;
     }
     if (bad) {   // uniform over the workgroup
@@ -790,9 +862,9 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(WAVE
       continue;
     }
     const int nmb = (rows + 15) >> 4;
-#define MOE_GITEM(M)                                                                      \
-  grouped_item<M, D, F, PBIAS, NB, WAVES, GU>(pa, aq, ars, k, perm, ref, r0, rows, nb0, h_out, \
-                                              rs_out, scores, yp, act, alpha, limit, L)
+#define MOE_GITEM(M)                                                                          \
+  grouped_item<M, CB, D, F, PBIAS, GU>(pa, aq, ars, tok, perm, ref, r0, rows, nb0, h_out, \
+                                       rs_out, scores, yp, act, alpha, limit, L)
     if (nmb == 1) MOE_GITEM(1);
     else if (nmb == 2) MOE_GITEM(2);
     else if (nmb == 3) MOE_GITEM(3);
@@ -800,6 +872,35 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(WAVE
 #undef MOE_GITEM
     __syncthreads();   // the LDS of this item is read before the next item stages
   }
+}
+
+// CBW column blocks per wave and projection when the call has at least
+// kWideItems such items, CBN otherwise
+template <int D, int F, bool PBIAS, int CBW, int CBN, bool GU>
+__global__ __launch_bounds__(kMmThreads) __attribute__((amdgpu_waves_per_eu(2))) void
+grouped_mm_kernel(PoolArgs pa, const uint16_t *__restrict__ aq, const uint16_t *__restrict__ ars,
+                  TokenOf tok, const int32_t *__restrict__ perm,
+                  const int4 *__restrict__ tiles, const int32_t *__restrict__ n_tiles,
+                  uint16_t *__restrict__ h_out, uint16_t *__restrict__ rs_out,
+                  const float *__restrict__ scores, float *__restrict__ yp, int act, float alpha,
+                  float limit) {
+  constexpr int NOUT = GU ? F : D, NBW = 16 * CBW * kMmWaves;
+  constexpr int NW = CBW * (GU ? 2 : 1);
+  __shared__ uint4 a_l[4 * kTileM * 8];
+  static_assert(NW <= 4, "code region");
+  __shared__ uint4 b_l[kMmWaves * kCodeBytes / 16];
+  // (a fragment read of the last row may run past it)
+  __shared__ uint4 s_l[kMmWaves * NW * GDim<GU ? D : F>::SPB + 1];
+  __shared__ int rp_l[GU ? 1 : kTileM];
+  __shared__ float rc_l[GU ? 1 : kTileM];
+  const GLds L{a_l, reinterpret_cast<char *>(b_l), reinterpret_cast<char *>(s_l), rp_l, rc_l};
+  const int nt = *n_tiles;
+  if (nt * ((NOUT + NBW - 1) / NBW) >= kWideItems)
+    grouped_items<CBW, D, F, PBIAS, GU>(pa, aq, ars, tok, perm, tiles, nt, h_out, rs_out,
+                                        scores, yp, act, alpha, limit, L);
+  else
+    grouped_items<CBN, D, F, PBIAS, GU>(pa, aq, ars, tok, perm, tiles, nt, h_out, rs_out,
+                                        scores, yp, act, alpha, limit, L);
 }
 
 // y[t, :] = sum over ranks r (ascending) of Yp[t*k + r, :]; 4 outputs/thread
@@ -826,35 +927,33 @@ __global__ __launch_bounds__(256) void combine_pairs_kernel(
 }
 
 // ---------------------------------------------------------------------------
-template <int D, int F, bool PB, int NBU, int WU>
+template <int D, int F, bool PB, int CBW, int CBN>
 static void launch_gg(dim3 g, hipStream_t s, const PoolArgs &pa, const uint16_t *xq,
-                      const float *rsx, int k, const int32_t *perm, const int4 *tiles,
-                      const int32_t *nt, uint16_t *h, float *rsh, int act, float alpha,
+                      const uint16_t *rsx, int k, const int32_t *perm, const int4 *tiles,
+                      const int32_t *nt, uint16_t *h, uint16_t *rsh, int act, float alpha,
                       float limit) {
-  hipLaunchKernelGGL((grouped_mm_kernel<D, F, PB, NBU, WU, true>), g, dim3(64 * WU), 0, s, pa,
-                     xq, rsx, k, perm, tiles, nt, h, rsh, nullptr, nullptr, act, alpha, limit);
+  hipLaunchKernelGGL((grouped_mm_kernel<D, F, PB, CBW, CBN, true>), g, dim3(kMmThreads), 0, s, pa,
+                     xq, rsx, token_of(k), perm, tiles, nt, h, rsh, nullptr, nullptr, act, alpha,
+                     limit);
 }
-template <int D, int F, bool PB, int NBD, int WD>
+template <int D, int F, bool PB, int CBW, int CBN>
 static void launch_gd(dim3 g, hipStream_t s, const PoolArgs &pa, const uint16_t *hq,
-                      const float *rsh, const float *sc, const int32_t *perm,
+                      const uint16_t *rsh, const float *sc, const int32_t *perm,
                       const int4 *tiles, const int32_t *nt, float *yp) {
-  hipLaunchKernelGGL((grouped_mm_kernel<D, F, PB, NBD, WD, false>), g, dim3(64 * WD), 0, s,
-                     pa, hq, rsh, 1, perm, tiles, nt, nullptr, nullptr, sc, yp, 0, 0.f, 0.f);
+  hipLaunchKernelGGL((grouped_mm_kernel<D, F, PB, CBW, CBN, false>), g, dim3(kMmThreads), 0, s,
+                     pa, hq, rsh, token_of(1), perm, tiles, nt, nullptr, nullptr, sc, yp, 0, 0.f, 0.f);
 }
 
-// (features per work item, waves) of gate/up and of down per geometry.  Only
-// these shapes are validated (the grouped parity tests with tiles of 1 to 64
-// rows); another shape that compiles is not known to be correct (down at
-// (64, 4) was measured wrong at 64-row tiles).
-#define MOE_GROUPED_GEOM(D, F, PB, NBU, WU, NBD, WD)                                     \
-  {D, F, PB, NBU, NBD, &launch_gg<D, F, PB, NBU, WU>, &launch_gd<D, F, PB, NBD, WD>}
+// column blocks per wave (many items, few items) of gate/up and of down
+#define MOE_GROUPED_GEOM(D, F, PB)                                                         \
+  {D, F, PB, 64, 128, &launch_gg<D, F, PB, 2, 1>, &launch_gd<D, F, PB, 4, 2>}
 static const GroupedLaunch kGroupedTable[] = {
-    MOE_GROUPED_GEOM(2048, 768, false, 64, 4, 128, 8),   // Qwen3-30B-A3B
-    MOE_GROUPED_GEOM(2048, 768, true, 64, 4, 128, 8),
-    MOE_GROUPED_GEOM(2880, 2880, true, 96, 6, 192, 6),   // gpt-oss-120b
-    MOE_GROUPED_GEOM(2880, 2880, false, 96, 6, 192, 6),
-    MOE_GROUPED_GEOM(256, 128, false, 128, 8, 128, 8),   // small test geometry
-    MOE_GROUPED_GEOM(256, 128, true, 128, 8, 128, 8),
+    MOE_GROUPED_GEOM(2048, 768, false),   // Qwen3-30B-A3B
+    MOE_GROUPED_GEOM(2048, 768, true),
+    MOE_GROUPED_GEOM(2880, 2880, true),   // gpt-oss-120b
+    MOE_GROUPED_GEOM(2880, 2880, false),
+    MOE_GROUPED_GEOM(256, 128, false),    // small test geometry
+    MOE_GROUPED_GEOM(256, 128, true),
 };
 
 const GroupedLaunch *find_grouped(int d_model, int d_ff, int has_bias) {
@@ -872,25 +971,24 @@ GroupedWs grouped_ws(int64_t T, int k, int D, int F) {
   w.off_perm = o; o += al((size_t)P * 4);
   w.off_tiles = o; o += al((size_t)w.max_tiles * 16);
   w.off_ntiles = o; o += al(4);
-  w.off_h = o; o += al((size_t)P * F * 2);
   w.off_yp = o; o += al((size_t)P * D * 4);
   w.off_xq = o; o += al((size_t)T * D * 2);
-  w.off_rsx = o; o += al((size_t)T * (D / 64) * 4);
+  w.off_rsx = o; o += al((size_t)T * 3 * rs_pitch(D) * 2);
   w.off_hq = o; o += al((size_t)P * F * 2);
-  w.off_rsh = o; o += al((size_t)P * (F / 64) * 4);
+  w.off_rsh = o; o += al((size_t)P * 3 * rs_pitch(F) * 2);
   w.total = o;
   return w;
 }
 
 // (in launches of at most 2^30 pieces, so the kernel's indices fit 32 bits)
-static void launch_prep(const uint16_t *src, int64_t rows, int K, uint16_t *dst, float *rs,
+static void launch_prep(const uint16_t *src, int64_t rows, int K, uint16_t *dst, uint16_t *rs,
                         hipStream_t s) {
   const int64_t chunk = ((int64_t)1 << 30) / (K / 8);
   for (int64_t r0 = 0; r0 < rows; r0 += chunk) {
     const int64_t nr = std::min(chunk, rows - r0);
     const int64_t n = nr * (K / 8);
     hipLaunchKernelGGL(grouped_prep_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s,
-                       src + r0 * K, nr, K, dst + r0 * K, rs + r0 * (K / 64));
+                       src + r0 * K, nr, K, dst + r0 * K, rs + r0 * 3 * rs_pitch(K));
   }
 }
 
@@ -903,12 +1001,11 @@ void launch_grouped(const GroupedLaunch *G, const PoolArgs &pa, const int32_t *r
   int32_t *perm = reinterpret_cast<int32_t *>(ws + w.off_perm);
   int4 *tiles = reinterpret_cast<int4 *>(ws + w.off_tiles);
   int32_t *ntiles = reinterpret_cast<int32_t *>(ws + w.off_ntiles);
-  uint16_t *h = reinterpret_cast<uint16_t *>(ws + w.off_h);
   float *yp = reinterpret_cast<float *>(ws + w.off_yp);
   uint16_t *xq = reinterpret_cast<uint16_t *>(ws + w.off_xq);
-  float *rsx = reinterpret_cast<float *>(ws + w.off_rsx);
+  uint16_t *rsx = reinterpret_cast<uint16_t *>(ws + w.off_rsx);
   uint16_t *hq = reinterpret_cast<uint16_t *>(ws + w.off_hq);
-  float *rsh = reinterpret_cast<float *>(ws + w.off_rsh);
+  uint16_t *rsh = reinterpret_cast<uint16_t *>(ws + w.off_rsh);
   const int nkeys = pa.n_slots + pa.n_records;
   const int64_t xpieces = (int64_t)T * (D / 8);
   if (xpieces < ((int64_t)1 << 30)) {   // grouping and x prep in one launch
@@ -920,13 +1017,14 @@ void launch_grouped(const GroupedLaunch *G, const PoolArgs &pa, const int32_t *r
                        pa.n_slots, pa.n_records, D, perm, tiles, ntiles, yp);
     launch_prep(x, T, D, xq, rsx, s);
   }
-  const int64_t items_up = w.max_tiles * (F / G->nb_up), items_down = w.max_tiles * (D / G->nb_down);
-  const bool fused = G->nb_up % 64 == 0;   // gate/up writes hq and rsh itself
-  G->gate_up(dim3((unsigned)std::min<int64_t>(items_up, kGroupedMaxWGs)), s, pa, xq, rsx, k, perm,
-             tiles, ntiles, fused ? hq : h, fused ? rsh : nullptr, act, alpha, limit);
-  if (!fused) launch_prep(h, P, F, hq, rsh, s);
-  G->down(dim3((unsigned)std::min<int64_t>(items_down, kGroupedMaxWGs)), s, pa, hq, rsh, scores,
-          perm, tiles, ntiles, yp);
+  // (at most one partial tile per slot reference in use)
+  const int64_t max_tiles = std::min<int64_t>(P, nkeys) + P / kTileM;
+  auto grid = [&](int nout, int nb) {
+    const int64_t items = (max_tiles + 7) / 8 * 8 * ((nout + nb - 1) / nb);
+    return dim3((unsigned)std::min<int64_t>(items, kGroupedMaxWGs));
+  };
+  G->gate_up(grid(F, G->nb_up), s, pa, xq, rsx, k, perm, tiles, ntiles, hq, rsh, act, alpha, limit);
+  G->down(grid(D, G->nb_down), s, pa, hq, rsh, scores, perm, tiles, ntiles, yp);
   const int64_t n4 = (int64_t)T * D / 4;
   hipLaunchKernelGGL(combine_pairs_kernel, dim3((unsigned)((n4 + 255) / 256)), dim3(256), 0,
                      s, yp, T, k, D, out, out32);

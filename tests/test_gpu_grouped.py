@@ -368,3 +368,32 @@ def test_multi_token_stack_graph_replays_equal_eager(T, block, expect):
     assert torch.equal(y, st.y[Lx])
     del st
     torch.cuda.empty_cache()
+
+
+@pytest.mark.parametrize("geom,T", [(G.QWEN3_30B_A3B, 2560), (G.GPT_OSS_120B, 1024)],
+                         ids=["qwen3", "gptoss"])
+def test_grouped_wide_items_equal_narrow_items(geom, T):
+    """A call of enough tiles for the wide work items (2,048 of them: 128 of
+    Qwen3's gate/up features or 256 outputs each) gives the rows of calls that
+    take the narrow ones, bit for bit: tiles of 1 to 64 rows, the last feature
+    block of gpt-oss partly past the matrix."""
+    layer = Layer(geom, geom.n_experts + 8, seed=20260071, router_bias=True)
+    rng = np.random.default_rng(20260072)
+    # experts of every row-block count: popularity from 1 to 200 rows a tile list
+    p = np.linspace(0.05, 1.0, geom.n_experts)
+    z = np.log(p) + rng.gumbel(size=(T, geom.n_experts))
+    ids = np.argpartition(-z, geom.top_k - 1, axis=1)[:, :geom.top_k]
+    n_tiles = sum(-(-c // 64) for c in np.bincount(ids.ravel(), minlength=geom.n_experts))
+    assert n_tiles * (-(-geom.d_ff // 128)) >= 2048
+    refs = layer.table[torch.tensor(ids, device="cuda")].to(torch.int32).contiguous()
+    scores = torch.tensor(rng.dirichlet(np.ones(geom.top_k), T).astype(np.float32), device="cuda")
+    x = bf16_randn((T, geom.d_model), seed=20260073)
+    y = torch.zeros((T, geom.d_model), dtype=torch.float32, device="cuda")
+    ops.ffn_grouped(layer.pool, refs, scores, x, out_f32=y)
+    for n in (7, 97):
+        yn = torch.zeros((n, geom.d_model), dtype=torch.float32, device="cuda")
+        ops.ffn_grouped(layer.pool, refs[:n].contiguous(), scores[:n].contiguous(),
+                        x[:n].contiguous(), out_f32=yn)
+        torch.cuda.synchronize()
+        ops.check_device_error()
+        assert torch.equal(yn, y[:n]), n
