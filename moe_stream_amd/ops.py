@@ -191,11 +191,17 @@ class RouteBuffers:
     """Device outputs of one routing call for T tokens."""
 
     def __init__(self, T: int, k: int, k_pred: int, device):
-        self.ids = torch.zeros((T, k), dtype=torch.int32, device=device)
-        self.scores = torch.zeros((T, k), dtype=torch.float32, device=device)
-        self.pred = torch.zeros((T, max(k_pred, 1)), dtype=torch.int32, device=device)
-        self.slot_refs = torch.zeros((T, k), dtype=torch.int32, device=device)
-        self.miss = torch.zeros((1,), dtype=torch.int32, device=device)
+        # one zeroed allocation, each output at a 16-byte boundary: an
+        # allocation and a fill kernel per output were most of a one-token
+        # routing call's time when the caller keeps no buffers
+        kp = max(k_pred, 1)
+        a, b = -(-T * k // 4) * 4, -(-T * kp // 4) * 4
+        m = torch.zeros(3 * a + b + 1, dtype=torch.int32, device=device)
+        self.ids = m[:T * k].view(T, k)
+        self.scores = m[a:a + T * k].view(torch.float32).view(T, k)
+        self.slot_refs = m[2 * a:2 * a + T * k].view(T, k)
+        self.pred = m[3 * a:3 * a + T * kp].view(T, kp)
+        self.miss = m[3 * a + b:]
 
 
 def route(x: torch.Tensor, W: torch.Tensor, bias: torch.Tensor | None, mode: int,
