@@ -339,27 +339,6 @@ __device__ __forceinline__ uint4 lds_frag(const char *p, int v) {
   return keep_halves(make_uint4(a.x, a.y, b.x, b.y), v);
 }
 
-// sigmoid in fp32, about 2 ulp: exp(-x) as exp2 of the product's leading part
-// with its remainder applied to first order, and one Newton step on the
-// reciprocal (of expf and the division it takes a third of the instructions;
-// the activation is a fifth of a full tile's VALU work).  Past +-87 it is 1 or
-// 2^-126 to within fp32's range.
-__device__ __forceinline__ float sigmoid_f32(float x) {
-  x = fminf(fmaxf(x, -87.f), 87.f);
-  const float hi = x * -1.44269502f;                        // -log2(e), leading part
-  const float lo = fmaf(x, -1.44269502f, -hi) + x * -1.92596303e-8f;
-  float e = __builtin_amdgcn_exp2f(hi);
-  e = fmaf(e, lo * 0.693147181f, e);
-  const float d = 1.f + e, r = __builtin_amdgcn_rcpf(d);
-  return fmaf(fmaf(-d, r, 1.f), r, r);
-}
-__device__ __forceinline__ float gated_act(int act, float g, float u, float alpha, float limit) {
-  if (act == MOE_ACT_SWIGLU) return g * sigmoid_f32(g) * u;
-  g = fminf(g, limit);
-  u = fminf(fmaxf(u, -limit), limit);
-  return g * sigmoid_f32(alpha * g) * (u + 1.f);
-}
-
 struct GLds {
   uint4 *a;                    // two buffers of [groups][row * 8 + (piece ^ (row & 7))]
   char *b;                     // [4 waves][N blocks][16 rows][64 bytes], swizzled
@@ -774,7 +753,7 @@ __device__ __forceinline__ void grouped_item(
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
           const int rr = rb * 16 + 4 * kq + e;
-          const float hv = gated_act(act, acc[rb][cb][0][e] + pb[0][cb],
+          const float hv = apply_act(act, acc[rb][cb][0][e] + pb[0][cb],
                                      acc[rb][cb][NPROJ - 1][e] + pb[NPROJ - 1][cb], alpha, limit);
           tile[rr * NB + (npl ^ swz(rr))] = (uint16_t)f32_to_bf16(hv);
         }

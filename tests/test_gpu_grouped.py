@@ -9,6 +9,7 @@ import torch
 
 from moe_stream_amd import _lib, ops, synth
 from moe_stream_amd import geometry as G
+from moe_stream_amd.pool import SlotPool
 from oracle import numerics as N
 
 from helpers import TOL, Layer, bf16_bits, bf16_randn, bf16_values
@@ -397,3 +398,62 @@ def test_grouped_wide_items_equal_narrow_items(geom, T):
         torch.cuda.synchronize()
         ops.check_device_error()
         assert torch.equal(yn, y[:n]), n
+
+
+def _plain_records(geom, n, parts):
+    """n store records, zero but for parts[component name]: bf16 values
+    broadcast over [n, *component shape], or code words."""
+    rec = torch.zeros((n, geom.record_bytes), dtype=torch.uint8, device="cuda")
+    for name, v in parts.items():
+        c = geom.comp(name)
+        dt = torch.int32 if c.dtype == "U32" else torch.bfloat16
+        full = v.to(dt).expand((n, *c.shape)).contiguous()
+        rec[:, c.offset:c.offset + c.nbytes].copy_(full.view(n, -1).view(torch.uint8))
+    return rec
+
+
+@pytest.mark.parametrize("act", [_lib.MOE_ACT_SWIGLU, _lib.MOE_ACT_SWIGLU_CLAMP])
+def test_grouped_activation_far_gates(act):
+    """Gates far outside the sigmoid's range give what the activation's formula
+    and the decode kernels give: zero far below, the gate (or its limit) far
+    above.  Expert e has gate value g[e] and up value u in one feature and zeros
+    elsewhere, and passes it on: with x = 1/256 the gate is its quant bias times
+    the sum of x, which is 1."""
+    geom = G.SMALL.with_(act=act)
+    g = [-3.3e38, -1e30, -1e8, -1e5, -1000.0, -104.0, -89.0, -80.0,
+         -20.0, -3.0, 0.0, 5.0, 30.0, 100.0, 1e8, 1e30]
+    g = torch.tensor(g, dtype=torch.bfloat16, device="cuda")
+    assert g.numel() == geom.n_experts
+    E, F, u = geom.n_experts, geom.d_ff, 3.0
+    one = torch.zeros((F, 1), device="cuda")
+    one[5] = 1.0
+    gate = torch.zeros((E, F, 1), device="cuda", dtype=torch.bfloat16)
+    gate[:, 5, 0] = g
+    down = torch.tensor([1.0, 0.0], device="cuda")   # outputs: the first group's sum
+    # (the clamped form multiplies by u + 1, so its other features need u = -1)
+    up = u * one - (0.0 if act == _lib.MOE_ACT_SWIGLU else 1.0) * (1.0 - one)
+    rec = _plain_records(geom, E, {"gate_proj.biases": gate, "up_proj.biases": up,
+                                   "down_proj.biases": down})
+    pool = SlotPool(geom, 1, "cuda", store=rec)
+    refs = (-1 - torch.arange(E, dtype=torch.int32, device="cuda")).view(E, 1)
+    sc = torch.ones((E, 1), device="cuda")
+    x = torch.full((E, geom.d_model), 1.0 / 256, dtype=torch.bfloat16, device="cuda")
+    y = ops.ffn_grouped(pool, refs, sc, x, out_f32=torch.empty(x.shape, device="cuda"))
+    yd = torch.empty(x.shape, device="cuda")
+    for e in range(E):
+        ops.ffn_decode(pool, refs[e:e + 1], sc[e:e + 1], x[e:e + 1], out_f32=yd[e:e + 1])
+    torch.cuda.synchronize()
+    ops.check_device_error()
+    v = g.double()
+    if act == _lib.MOE_ACT_SWIGLU:
+        want = v * torch.sigmoid(v) * u
+    else:
+        v = v.clamp(max=geom.limit)
+        want = v * torch.sigmoid(geom.alpha * v) * (u + 1)
+    for got in (y, yd):
+        got = got[:, :1].double().squeeze(1)
+        # h is bf16, 8 significant bits: 2^-8 of its value at most, and fp32's
+        # exp; below -88.7 that is infinite and h zero, where the true value is
+        # under 89 e^-88.7 (u + 1)
+        ok = (got - want).abs() <= want.abs() * (2.0 ** -8 + 1e-5) + 1.1e-36
+        assert bool(ok.all()), torch.stack([got, want])
