@@ -10,12 +10,16 @@
 //   combine_pairs      : y[t] = sum over ranks r of Yp[t*k + r] (rank order)
 //
 // Dequantisation rides on the MFMA.  A word of eight 4-bit codes becomes a
-// B fragment of bf16 values 128+q (exact, one v_bfi_b32 per pair), each
+// B fragment of bf16 values 128+q (exact, one v_and_or_b32 per pair), each
 // 64-input quant group accumulates into a fresh accumulator, and
 //   out += S * acc + (B - 128*S) * rowsum(X over the group),
 // the factorised group form of kernels.py:141-145, with exact products and
-// fp32 accumulation.  The 8 inputs of one MFMA lane are permuted identically
-// in A and B (x_pairs order), which leaves every dot product unchanged.
+// fp32 accumulation.  The second term is added every 4 groups, so the 128 offset
+// cancels there and is not carried through the row (relative rms error of the sums
+// against 64 bits, fp32 emulation: 1.8e-6 at 768, 2,048 and 2,880 inputs of mean
+// zero, 4e-6 to 5e-6 of mean one; with the whole row's term added at once 2.9e-6,
+// 4.3e-6 and 5.1e-6, and 3e-5 to 4e-5).  The 8 inputs of one MFMA lane are permuted
+// identically in A and B (x_pairs order), which leaves every dot product unchanged.
 //
 // Every output row is one dot product per feature, computed by exactly one
 // tile with a fixed accumulation order, so results do not depend on how the
@@ -168,27 +172,20 @@ __global__ __launch_bounds__(1024) void group_pairs_kernel(
   group_pairs_body(refs, n_pairs, n_slots, n_records, D, perm, tiles, n_tiles, yp);
 }
 
-// The fp32 sum of a row's group g as three bf16 parts whose sum is exact (3 x 8
-// significant bits): lane m < 3 of those that hold the sum writes part m.
-// row: [3][pitch], the pitch the groups rounded up to 32.
-__host__ __device__ constexpr int rs_pitch(int K) { return (K / 64 + 31) / 32 * 32; }
-__device__ __forceinline__ void put_row_sum(uint16_t *row, int pitch, int g, int m, float x) {
-  const float p0 = round_bf16(x), r = x - p0, p1 = round_bf16(r);
-  if (m < 3) row[m * pitch + g] = (uint16_t)f32_to_bf16(m == 0 ? p0 : m == 1 ? p1 : r - p1);
-}
+// Row sums: fp32, a row's groups padded to a multiple of 4 (16-byte rows).
+__host__ __device__ constexpr int rs_pitch(int K) { return (K / 64 + 3) / 4 * 4; }
 
 // ---------------------------------------------------------------------------
 // The A operand's rows in x_pairs order (each 8-input piece p holds inputs
 // (0,4), (1,5), (2,6), (3,7) pairwise, the order of the B fragments) and their
 // 64-input row sums, once per call: one thread per piece, the 8 pieces of a
-// group in 8 consecutive lanes (rs: [rows][3][rs_pitch(K)] bf16, see
-// put_row_sum).
+// group in 8 consecutive lanes (rs: [rows][rs_pitch(K)] fp32).
 // ---------------------------------------------------------------------------
 // piece i of `rows` rows of K inputs (32-bit index arithmetic: the host
 // passes at most 2^30 pieces at a time)
 __device__ __forceinline__ void prep_piece(int i, const uint16_t *__restrict__ src, int64_t rows,
                                            int K, uint16_t *__restrict__ dst,
-                                           uint16_t *__restrict__ rs) {
+                                           float *__restrict__ rs) {
   const int ppr = K / 8;
   const bool ok = i < (int)(rows * ppr);
   const int r = ok ? i / ppr : 0;
@@ -204,14 +201,14 @@ __device__ __forceinline__ void prep_piece(int i, const uint16_t *__restrict__ s
   sm = group_sum<8>(sm);
   if (ok) {
     *reinterpret_cast<uint4 *>(dst + (int64_t)r * K + pc * 8) = make_uint4(out[0], out[1], out[2], out[3]);
-    put_row_sum(rs + (int64_t)r * (3 * rs_pitch(K)), rs_pitch(K), pc / 8, pc & 7, sm);
+    if ((pc & 7) == 0) rs[(int64_t)r * rs_pitch(K) + pc / 8] = sm;
   }
 }
 
 __global__ __launch_bounds__(256) void grouped_prep_kernel(const uint16_t *__restrict__ src,
                                                            int64_t rows, int K,
                                                            uint16_t *__restrict__ dst,
-                                                           uint16_t *__restrict__ rs) {
+                                                           float *__restrict__ rs) {
   prep_piece(blockIdx.x * 256 + threadIdx.x, src, rows, K, dst, rs);
 }
 
@@ -221,7 +218,7 @@ __global__ __launch_bounds__(1024) void group_prep_kernel(
     const int32_t *__restrict__ refs, int n_pairs, int n_slots, int n_records, int D,
     int32_t *__restrict__ perm, int4 *__restrict__ tiles, int32_t *__restrict__ n_tiles,
     float *__restrict__ yp, const uint16_t *__restrict__ x, int64_t T, uint16_t *__restrict__ xq,
-    uint16_t *__restrict__ rsx) {
+    float *__restrict__ rsx) {
   if (blockIdx.x == 0)
     group_pairs_body(refs, n_pairs, n_slots, n_records, D, perm, tiles, n_tiles, yp);
   else
@@ -250,26 +247,25 @@ __global__ __launch_bounds__(1024) void group_prep_kernel(
 //    8-byte piece costs a cache access of its own.)
 //  * Each group accumulates into a fresh 16x16 block (2 MFMAs over the bf16
 //    128+q codes), folded into the output by S.
-//  * The scale rows sit in LDS for the whole item (read 8 bytes at a time from
-//    memory they cost a cache line per row and quad).
-//  * The bias term sum_g rowsum[g] * (B[g] - 128 S[g]) starts the output
-//    block: three bf16 MFMAs of the row sums' parts against the B row and three
-//    against the S row (the record's own bf16 values) give it with exact
-//    products and fp32 sums.
+//  * The scale and bias rows come 16 groups at a time (32 bytes of a row), a chunk
+//    ahead through registers into a region of the wave's own, the row sums are in
+//    LDS for the whole item.
+//  * The bias term sum_g rowsum[g] * (B[g] - 128 S[g]): per quad and block one
+//    fp32 MFMA of K = 4 groups from zero, added behind the quad's folds.  (The fp32
+//    MFMA takes two of the bf16 ones' time, an eighth of a quad's; bf16 ones over
+//    the sums in three parts are cheaper but have no exact B - 128 S to work on.)
 //
-// Measured (whole block against the previous kernels: 64-row tiles with codes and
-// rows staged a quad at a time behind two barriers, the bias term on fp32 MFMAs;
-// cold weights): Qwen3 4,096 tokens 698 -> 585 us, gpt-oss 700 tokens 747 -> 640,
-// gpt-oss 29 tokens 210 -> 166.  A full gate/up tile now spends 30 of its 44 us in
-// the quads, two waves per SIMD at about half the MFMA rate; the rest is the first
-// operands' latency and the epilogue.  One-block tiles are bound by HBM and that
-// latency.
+// Measured (whole block against the kernels before these: 64-row tiles with codes
+// and rows staged a quad at a time behind two barriers, narrow items only, cold
+// weights; results bit for bit the same): Qwen3 4,096 tokens 694 -> 587 us, 512
+// tokens 147 -> 145, gpt-oss 700 tokens 750 -> 605, 29 tokens 212 -> 178.
 //
 // What sets the shape: per group a wave's M x N blocks (N = CB * NPROJ) take
-// 32 M N matrix-core cycles, 64 M LDS cycles (a 16-row fragment is 2 KB, the
-// CU's LDS serves four SIMDs at 128 B/cycle) and 4 * (14 N + 4 M N) VALU cycles
-// (decode of 2 N code words, fold).  At M = 4 the LDS reads alone exceed the
-// MFMAs for N < 2; at N = 4 they are half of them and the VALU work is level.
+// 32 M N matrix-core cycles (8 M N more for the bias term), 64 M LDS cycles (a
+// 16-row fragment is 2 KB, the CU's LDS serves four SIMDs at 128 B/cycle) and
+// 4 * (14 N + 5 M N) VALU cycles (decode of 2 N code words, fold, bias term).  At
+// M = 4 the LDS reads alone exceed the MFMAs for N < 2; at N = 4 they are half of
+// them and the VALU work is level.
 // Rows past the tile compute garbage from a copy of a real row, which no
 // output row depends on (MFMA rows are independent) and nothing stores;
 // features past the matrix likewise (their addresses are clamped).
@@ -281,12 +277,10 @@ struct GDim {
   static constexpr int NG = KIN / 64;             // quant groups along the inputs
   static constexpr int NQ = (NG + 3) / 4;         // quads
   static constexpr int NGL = NG - 4 * (NQ - 1);   // groups of the last quad
-  // scale rows in LDS: as they are where a quad's 4 halfwords are then 8-byte
-  // aligned, else each padded to 16 bytes
-  static constexpr bool SRAW = NG % 4 == 0;
-  static constexpr int SPB = SRAW ? NG * 2 : (NG + 7) / 8 * 16;   // row pitch, bytes
-  static constexpr int SPP = SPB;                 // 16-byte pieces of a block's 16 rows
-  static constexpr int KS = (NG + 31) / 32;       // bias MFMA steps (32 groups each)
+  // scales and biases in LDS: 16 groups (a chunk, 32 bytes of a row) at a time
+  static constexpr int NCH = (NQ + 3) / 4;        // chunks
+  // row sums in LDS: the 16 rows of a fragment on distinct banks (pitch 4 x odd)
+  static constexpr int RP = rs_pitch(KIN), RSP = RP % 8 ? RP : RP + 4;
   static_assert(KIN % 64 == 0, "whole quant groups");
 };
 
@@ -297,18 +291,13 @@ __device__ __forceinline__ uint32_t gload2(const void *p) {
   return *(const __attribute__((address_space(1))) uint16_t *)(p);
 }
 
-// keeps halfwords [0, v) of a 16-byte fragment
-__device__ __forceinline__ uint4 keep_halves(uint4 f, int v) {
-  auto m = [&](int w) { return 2 * w + 1 < v ? 0xffffffffu : 2 * w < v ? 0xffffu : 0u; };
-  return make_uint4(f.x & m(0), f.y & m(1), f.z & m(2), f.w & m(3));
-}
-
-// Chunk ci of a row of NG (odd or small) bf16 values, 2-byte aligned: halfwords
-// 8 ci .. + 7, zero past NG.  The load never leaves the row's dwords (a window
-// across the row's end is read 8 halfwords before it and shifted) and is
-// dword-aligned: a 16-byte load at an odd halfword takes several times as long.
+// Chunk ci of a row of NG bf16 values: halfwords 8 ci .. + 7, zero past NG.  The
+// load never leaves the row's dwords (a window across the row's end is read 8
+// halfwords before it and shifted) and is dword-aligned: a 16-byte load at an odd
+// halfword takes several times as long.
 template <int NG>
 __device__ __forceinline__ uint4 row_chunk(const char *row, int ci) {
+  if (NG % 8 == 0) return gload16(row + 16 * ci);
   if (NG < 8) {
     uint32_t h[8];
 #pragma unroll
@@ -319,10 +308,10 @@ __device__ __forceinline__ uint4 row_chunk(const char *row, int ci) {
   constexpr int SH = 8 - NG % 8;   // of the window across the end
   const int b = 8 * ci;
   const char *p = row + min(b, NG - 8) * 2;
-  const uint32_t odd = (uint32_t)(uintptr_t)p & 2u;
+  const uint32_t odd = NG % 2 ? (uint32_t)(uintptr_t)p & 2u : 0u;   // (even: rows of dwords)
   const char *p4 = p - odd;
   const u32x4_t f = *(const __attribute__((address_space(1))) u32x4_a4_t *)(p4);
-  const uint32_t l = (uint32_t)gload4i(p4 + (odd ? 16 : 12));
+  const uint32_t l = NG % 2 ? (uint32_t)gload4i(p4 + (odd ? 16 : 12)) : 0u;
   const uint32_t x[5] = {f.x, f.y, f.z, f.w, l};
   uint32_t w[8] = {0, 0, 0, 0, 0, 0, 0, 0}, t[4];
 #pragma unroll
@@ -333,16 +322,36 @@ __device__ __forceinline__ uint4 row_chunk(const char *row, int ci) {
   return b > NG - 8 ? make_uint4(t[0], t[1], t[2], t[3]) : make_uint4(w[0], w[1], w[2], w[3]);
 }
 
-// Fragment of 8 halfwords of a scale row in LDS (8-byte aligned)
-__device__ __forceinline__ uint4 lds_frag(const char *p, int v) {
-  const uint2 a = reinterpret_cast<const uint2 *>(p)[0], b = reinterpret_cast<const uint2 *>(p)[1];
-  return keep_halves(make_uint4(a.x, a.y, b.x, b.y), v);
+// Keeps the value's computation here in program order (emits nothing).
+template <class T>
+__device__ __forceinline__ void pin(T &v) {
+  asm volatile("" : "+v"(v));
+}
+
+// The sum of a row's 64 activations, 8 in x_pairs order in each of 8 consecutive
+// lanes (the lane of the first 8 has it).  Two orders of equal depth: each geometry
+// keeps the one that its results have always been computed with, prep_piece's where
+// d_ff is no multiple of 128 (there a kernel of its own took the sums).
+template <int F>
+__device__ __forceinline__ float h_row_sum(uint4 v) {
+  auto lo = [](uint32_t w) { return bf16_to_f32(w & 0xffffu); };
+  auto hi = [](uint32_t w) { return bf16_to_f32(w >> 16); };
+  const float a = (lo(v.x) + lo(v.y)) + (lo(v.z) + lo(v.w));
+  const float b0 = hi(v.x) + hi(v.y), b1 = hi(v.z) + hi(v.w);
+  if (F % 128) return group_sum<8>((a + b0) + b1);
+  // 16 features as a balanced tree, then the four of them in order
+  float s = a + (b0 + b1);
+  s += dpp_f<kDppQuadXor1>(s);
+  const float t = dpp_f<kDppQuadXor2>(s);   // (first lane: the second sum, ...)
+  return ((s + t) + dpp_f<kDppHalfMirror>(t)) + dpp_f<kDppHalfMirror>(s);
 }
 
 struct GLds {
   uint4 *a;                    // two buffers of [groups][row * 8 + (piece ^ (row & 7))]
   char *b;                     // [4 waves][N blocks][16 rows][64 bytes], swizzled
-  char *s;                     // [4 waves][N blocks][16 rows][SPB bytes]: the scales
+  char *s;                     // [4 waves][S, B][N blocks][16 rows][32 bytes]: a chunk
+  float *rs;                   // [64 rows][RSP]: the tile rows' sums
+  float *pb;                   // [4 waves][4 blocks][16]: the projection biases
   int *rperm;                  // down: the tile rows' pair ids [64] ...
   float *rsc;                  // ... and their scores [64]
 };
@@ -361,22 +370,16 @@ static TokenOf token_of(int k) {
   return {(uint32_t)((((uint64_t)1 << 32) + k - 1) / k), 0u};
 }
 
-// Keeps the value's computation here in program order (emits nothing).
-template <class T>
-__device__ __forceinline__ void pin(T &v) {
-  asm volatile("" : "+v"(v));
-}
-
 template <int M, int CB, int D, int F, bool PBIAS, bool GU>
 __device__ __forceinline__ void grouped_item(
-    const PoolArgs &pa, const uint16_t *__restrict__ aq, const uint16_t *__restrict__ ars,
+    const PoolArgs &pa, const uint16_t *__restrict__ aq, const float *__restrict__ ars,
     TokenOf tok, const int32_t *__restrict__ perm, int ref, int r0, int rows, int nb0,
-    uint16_t *__restrict__ h_out, uint16_t *__restrict__ rs_out,
+    uint16_t *__restrict__ h_out, float *__restrict__ rs_out,
     const float *__restrict__ scores, float *__restrict__ yp, int act, float alpha, float limit,
     const GLds &L) {
   constexpr int KIN = GU ? D : F, NOUT = GU ? F : D, NPROJ = GU ? 2 : 1;
   using I = GDim<KIN>;
-  constexpr int NG = I::NG, NQ = I::NQ, NGL = I::NGL, KS = I::KS, SPB = I::SPB;
+  constexpr int NG = I::NG, NQ = I::NQ, NGL = I::NGL;
   constexpr int NP = PBIAS ? 4 : 3, NB = 16 * CB * kMmWaves, RB = KIN / 2;
   constexpr int ROWS = 16 * M;
   // A in LDS: whole quads of 32 rows, or half quads of 64; R quads wait in
@@ -384,7 +387,11 @@ __device__ __forceinline__ void grouped_item(
   constexpr bool QA = M <= 2;
   constexpr int AROWS = QA ? 32 : 64, AG = QA ? 4 : 2, R = M == 1 ? 2 : 1;
   constexpr int SPG = AROWS * 8 / kMmThreads;   // A pieces per thread and group
-  const int tid = threadIdx.x, lane = tid & 63;
+  // (opaque here and at the epilogue: what hangs on it is computed there, not held
+  // in registers across the items or the quads)
+  int tid = threadIdx.x;
+  pin(tid);
+  const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int col = lane & 15, kq = lane >> 4;
   // (named, not arrays: a pointer picked from an array by a lane's index goes
@@ -407,11 +414,14 @@ __device__ __forceinline__ void grouped_item(
   if (!GU) pr_ep = row_index(lane);
   // codes of half a quad: lane l of a wave loads 16-byte chunk l & 3 of row l >>
   // 2 of each of its blocks
-  uint32_t boff[CB];
   const int bch = (lane & 3) * 16;
+  // first feature of column block cb (a block past the matrix: its last one)
+  auto block_f = [&](int cb) { return (uint32_t)min(nb0 + (wave * CB + cb) * 16, NOUT - 16); };
+  // (offsets per lane: as scalars they are spilled, 8 tokens through 12 layers 557 us
+  // against 548)
+  uint32_t boff[CB];
 #pragma unroll
-  for (int cb = 0; cb < CB; ++cb)
-    boff[cb] = (uint32_t)min(nb0 + (wave * CB + cb) * 16 + (lane >> 2), NOUT - 1) * RB;
+  for (int cb = 0; cb < CB; ++cb) boff[cb] = (block_f(cb) + (lane >> 2)) * RB;
   uint4 breg[R][2][N];   // codes to come
   auto load_b = [&](int q, int hf, int rs) {
     // (chunks past the row, in a last partial quad: its last one, unused)
@@ -419,8 +429,8 @@ __device__ __forceinline__ void grouped_item(
     const uint32_t c = RB % 64 == 0 || o + 64 <= RB ? (uint32_t)(o + bch)
                                                     : (uint32_t)min(o + bch, RB - 16);
 #pragma unroll
-    for (int n = 0; n < N; ++n) 
-      breg[rs][hf][n] = gload16((n % NPROJ ? w1 : w0) + boff[n / NPROJ] + c);
+    for (int n = 0; n < N; ++n)
+      breg[rs][hf][n] = gload16((n % NPROJ ? w1 : w0) + (boff[n / NPROJ] + c));
   };
   char *const bl = L.b + wave * kCodeBytes;
   const uint32_t bwr = (uint32_t)((lane >> 2) * 64 + (((lane & 3) ^ (lane >> 4)) << 4));
@@ -437,25 +447,36 @@ __device__ __forceinline__ void grouped_item(
   auto read_b = [&](int gi, int n) {
     return *reinterpret_cast<const uint2 *>(bl + n * 1024 + (brd ^ ((gi & 1) << 5)));
   };
-  // the wave's scale rows (and, for the bias term, bias rows), all of the
-  // item, as SPP 16-byte pieces per block of 16 rows (contiguous memory where
-  // the rows stay as they are, else a chunk of a row); a pass takes PB blocks (as
-  // many as fit the code region, which the bias rows pass through), lane l its
-  // pieces l, l + 64, ...
-  constexpr int SPP = I::SPP, PB = N * 16 * SPB <= kCodeBytes ? N : N / 2, NPASS = N / PB;
-  constexpr int NPC = PB * SPP, PT = (NPC + 63) / 64;
-  static_assert(PB >= 1 && PB * 16 * SPB <= kCodeBytes && N % PB == 0, "bias rows in the code region");
-  char *const sl = L.s + wave * (N * 16 * SPB);
-  auto scale_piece = [&](int h, int t, const char *a0, const char *a1) {
-    const int i = min(lane + 64 * t, NPC - 1), n = h * PB + i / SPP, o = i % SPP;
-    const int f = min(nb0 + (wave * CB + n / NPROJ) * 16, NOUT - 16);
-    const char *p = (NPROJ > 1 && (n & 1) ? a1 : a0) + (uint32_t)(f * (NG * 2));
-    if (I::SRAW) return gload16(p + o * 16);
-    return row_chunk<NG>(p + o / (SPB / 16) * (NG * 2), o % (SPB / 16));
+  // the wave's scale and bias rows a chunk at a time, as 16-byte pieces, SPT per lane
+  // and array: piece h = lane & 1 of row (lane >> 1) & 15 of block 2 t + (lane >> 5);
+  // in LDS at h ^ (row >> 3), so the 16 rows of an 8-byte read fall on distinct banks
+  constexpr int SPT = N / 2;
+  char *const sl = L.s + wave * (N * 1024);
+  auto load_s = [&](int ch, const char *b0, const char *b1, uint4 (&v)[SPT]) {
+    int ln = lane;
+    pin(ln);   // (the addresses are computed here each time)
+    const uint32_t row = (uint32_t)((ln >> 1) & 15) * (NG * 2);
+    // (pieces past the row: its last one, unused)
+    const int pc = min(2 * ch + (ln & 1), (NG - 1) / 8);
+#pragma unroll
+    for (int t = 0; t < SPT; ++t) {   // (block 2 t + 1: the other projection's, or the next)
+      const char *p0 = b0 + block_f(NPROJ > 1 ? t : 2 * t) * (NG * 2);
+      const char *p1 = b1 + block_f(NPROJ > 1 ? t : 2 * t + 1) * (NG * 2);
+      v[t] = row_chunk<NG>((ln & 32 ? p1 : p0) + row, pc);
+    }
   };
-  auto store_piece = [&](char *dst, int t, uint4 v) {   // into a pass's rows
-    const int i = lane + 64 * t;
-    if (NPC % 64 == 0 || i < NPC) *reinterpret_cast<uint4 *>(dst + i * 16) = v;
+  const uint32_t swr = (uint32_t)((lane >> 1) * 32 + (((lane & 1) ^ ((lane >> 4) & 1)) << 4));
+  auto store_s = [&](int arr, const uint4 (&v)[SPT]) {
+    asm volatile("" ::: "memory");
+#pragma unroll
+    for (int t = 0; t < SPT; ++t)
+      *reinterpret_cast<uint4 *>(sl + arr * (N * 512) + t * 1024 + swr) = v[t];
+    asm volatile("" ::: "memory");
+  };
+  // a row's 4 values (groups) of quad q
+  const uint32_t srd = (uint32_t)(col * 32 + ((col >> 3) << 4));
+  auto read_s = [&](int arr, int q, int n) {
+    return *reinterpret_cast<const uint2 *>(sl + (arr * N + n) * 512 + (srd ^ ((q & 3) << 3)));
   };
   // A: this thread's pieces of the rows (tid >> 3) + 32 j, half a quad at a time
   const uint16_t *asrc[SPG];
@@ -477,39 +498,27 @@ __device__ __forceinline__ void grouped_item(
         for (int j = 0; j < SPG; ++j)
           L.a[(buf * AG + i) * (AROWS * 8) + adst[j]] = areg[rs][i][j];
   };
-  // the scales, the first codes, the row sums' parts and the first A rows on
-  // their way
-  uint4 sv[NPASS][PT], bv[NPASS][PT];
-#pragma unroll
-  for (int h = 0; h < NPASS; ++h)
-#pragma unroll
-    for (int t = 0; t < PT; ++t) {
-      sv[h][t] = scale_piece(h, t, s0, s1);
-      bv[h][t] = scale_piece(h, t, o0, o1);
-    }
-  float pb[NPROJ][CB];
-#pragma unroll
-  for (int j = 0; j < NPROJ; ++j)
-#pragma unroll
-    for (int cb = 0; cb < CB; ++cb) {
-      pb[j][cb] = 0.f;
-      if (PBIAS) {
-        const int proj = GU ? (j == 0 ? PROJ_GATE : PROJ_UP) : PROJ_DOWN;
-        const int f = min(nb0 + (wave * CB + cb) * 16 + col, NOUT - 1);
-        pb[j][cb] =
-            bf16_to_f32(gload2(resolve(pa, comp_index(proj, PART_BIAS, NP), ref) + 2 * f));
-      }
-    }
+  // the first scales, biases and codes, the row sums and the first A rows on their way
+  uint4 sv[SPT], bv[SPT];
+  load_s(0, s0, s1, sv);
+  load_s(0, o0, o1, bv);
+  uint32_t pbv = 0;   // the projection bias of feature col of block kq
+  if (PBIAS) {
+    const char *const q0 = resolve(pa, comp_index(PF, PART_BIAS, NP), ref);
+    const char *const q1 = resolve(pa, comp_index(PL, PART_BIAS, NP), ref);
+    const int n = min(kq, N - 1);
+    const uint32_t f = (uint32_t)min(nb0 + (wave * CB + n / NPROJ) * 16, NOUT - 16) + col;
+    pbv = gload2((NPROJ > 1 && (n & 1) ? q1 : q0) + 2 * f);
+  }
   load_b(0, 0, 0);
   if (NG0 > 2) load_b(0, 1, 0);
-  constexpr int NGP = rs_pitch(KIN), RSP = 6 * NGP + 16, RSJ = 6 * NGP / 64;
-  static_assert(64 * RSP <= 4 * kTileM * 8 * 16, "row-sum parts in the A buffers");
+  constexpr int RPP = I::RP / 4, RSJ = (RPP + 3) / 4;   // 16-byte pieces of a row, per thread
   uint4 rsv[RSJ];
   {
     const int64_t row = GU ? tok(pr_rs) : r0 + min(tid >> 2, rows - 1);
-    const char *src = reinterpret_cast<const char *>(ars + row * (3 * NGP)) + (tid & 3) * 16;
+    const float *src = ars + row * I::RP;
 #pragma unroll
-    for (int i = 0; i < RSJ; ++i) rsv[i] = gload16(src + 64 * i);
+    for (int i = 0; i < RSJ; ++i) rsv[i] = gload16(src + 4 * min((tid & 3) + 4 * i, RPP - 1));
   }
 #pragma unroll
   for (int j = 0; j < SPG; ++j) {
@@ -530,51 +539,17 @@ __device__ __forceinline__ void grouped_item(
     L.rperm[lane] = pr_ep;
     L.rsc[lane] = gload4f(scores + pr_ep);
   }
+  store_s(0, sv);
+  store_s(1, bv);
+  if (PBIAS) L.pb[wave * 64 + lane] = bf16_to_f32(pbv);
 #pragma unroll
-  for (int h = 0; h < NPASS; ++h)
-#pragma unroll
-    for (int t = 0; t < PT; ++t) store_piece(sl + h * (PB * 16 * SPB), t, sv[h][t]);
-  {
-    char *const rl = reinterpret_cast<char *>(L.a) + (tid >> 2) * RSP + (tid & 3) * 16;
-#pragma unroll
-    for (int i = 0; i < RSJ; ++i) *reinterpret_cast<uint4 *>(rl + 64 * i) = rsv[i];
+  for (int i = 0; i < RSJ; ++i) {
+    const int p = (tid & 3) + 4 * i;
+    uint4 v = rsv[i];
+    if (NG % 4 && p == RPP - 1)   // (the pad meets a zero factor: it must be finite)
+      v = make_uint4(v.x, NG % 4 > 1 ? v.y : 0u, NG % 4 > 2 ? v.z : 0u, 0u);
+    if (p < RPP) *reinterpret_cast<uint4 *>(L.rs + (tid >> 2) * I::RSP + 4 * p) = v;
   }
-  __syncthreads();
-  // the output blocks start from the bias term
-#pragma unroll
-  for (int h = 0; h < NPASS; ++h) {
-    asm volatile("" ::: "memory");
-#pragma unroll
-    for (int t = 0; t < PT; ++t) store_piece(bl, t, bv[h][t]);
-    asm volatile("" ::: "memory");
-#pragma unroll
-    for (int i = 0; i < PB; ++i) {
-      const int n = h * PB + i, cb = n / NPROJ, j = n % NPROJ;
-#pragma unroll
-      for (int ks = 0; ks < KS; ++ks) {
-        // (chunks past the row: any, all zeroed)
-        const int ci = min(4 * ks + kq, (NG - 1) / 8), v = max(0, min(8, NG - (32 * ks + 8 * kq)));
-        const uint4 fs = lds_frag(sl + (n * 16 + col) * SPB + ci * 16, v);
-        const uint4 fb = lds_frag(bl + (i * 16 + col) * SPB + ci * 16, v);
-#pragma unroll
-        for (int rb = 0; rb < M; ++rb) {
-          const char *ra = reinterpret_cast<const char *>(L.a) + (rb * 16 + col) * RSP + ks * 64 + kq * 16;
-          f32x4_t cs = {0.f, 0.f, 0.f, 0.f};
-          f32x4_t &o = acc[rb][cb][j];
-#pragma unroll
-          for (int p = 0; p < 3; ++p) {
-            uint4 a = *reinterpret_cast<const uint4 *>(ra + p * 2 * NGP);
-            if (NG % 32) a = keep_halves(a, v);
-            o = mfma16x16x32(a, fb, o);
-            cs = mfma16x16x32(a, fs, cs);
-          }
-#pragma unroll
-          for (int e = 0; e < 4; ++e) o[e] -= 128.f * cs[e];
-        }
-      }
-    }
-  }
-  __syncthreads();   // the row-sum parts are read
   store_a(0, 0, NG0, 0);
   store_b(0, 0);
   // quads 1 .. R on their way (of the A rows whole quads only)
@@ -610,14 +585,38 @@ __device__ __forceinline__ void grouped_item(
   }
   S[1] = 0.f;
 #pragma unroll
-  for (int n = 0; n < N; ++n)
-    scur[n] = *reinterpret_cast<const uint2 *>(sl + (n * 16 + col) * SPB);
+  for (int n = 0; n < N; ++n) scur[n] = read_s(0, 0, n);
+  // The bias term of a quad, sum over its groups of rowsum * (B - 128 S): one fp32
+  // MFMA of K = 4 groups per block (A: row col, group kq; B: feature col, group kq)
+  // from zero, added behind the quad's folds, in the first group of the next quad:
+  // there the 128 offset of the codes cancels before it is carried any further.
+  float ra[M], C[N];
+  uint2 bnx = read_s(1, 0, 0);   // bias values to come
+  constexpr int BZ = M <= 2 ? M : 1;
+  f32x4_t bz[BZ];
+#pragma unroll
+  for (int rb = 0; rb < M; ++rb) ra[rb] = 0.f;
+#pragma unroll
+  for (int n = 0; n < N; ++n) C[n] = 0.f;
+  // halfword kq of 4 as an fp32 value
+  const uint32_t hsel = 0x01000c0cu + (uint32_t)kq * 0x02020000u;
+  auto pick = [&](uint2 v) { return __uint_as_float(__builtin_amdgcn_perm(v.y, v.x, hsel)); };
+  const float *const rsl = L.rs + col * I::RSP + kq;
+  auto bias_block = [&](int rb, int n) {
+    return __builtin_amdgcn_mfma_f32_16x16x4f32(ra[rb], C[n], (f32x4_t){0.f, 0.f, 0.f, 0.f}, 0, 0,
+                                                0);
+  };
+  auto add_block = [&](f32x4_t &o, const f32x4_t &v) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) o[e] += v[e];
+    pin(o);
+  };
   // fragment word m of 8, 4 of each code word, as pairs of bf16 128+q (one
-  // v_and_or_b32 after the shift: its constants in registers.  Not bfi_mask():
-  // the compiler does not see that an inline instruction writes a register
-  // that an MFMA in flight still reads)
+  // v_and_or_b32 after the shift: its constants in registers, one of them scalar.
+  // Not bfi_mask(): the compiler does not see that an inline instruction writes a
+  // register that an MFMA in flight still reads)
   uint32_t kmask = 0x000f000fu, kexp = 0x43004300u;
-  pin(kmask);
+  asm volatile("" : "+s"(kmask));
   pin(kexp);
   auto decode = [&](uint2 cw, int m) {
     return (((m < 4 ? cw.x : cw.y) >> (4 * (m & 3))) & kmask) | kexp;
@@ -626,29 +625,42 @@ __device__ __forceinline__ void grouped_item(
   creg[1] = read_b(1 / N, 1 % N);
 #pragma unroll
   for (int m = 0; m < 8; ++m) bf[0][m] = decode(creg[0], m);
-  // One quad of ng groups (constants, as is everything but q; par: its parity):
-  // steps s = gi * N + n, the step registers alternating by s.  Two steps
-  // before the end of each half, when the last of its codes are read, the next
-  // half's go from registers to the wave's own LDS and the loads of the same
-  // half R quads on are issued into the registers (ng_next, ng_second, ng_load:
-  // groups of quads q + 1, q + R and q + 1 + R, 0: none).  The A rows of the
-  // next quad go along with M <= 2, else half a quad ahead.  The barrier is one
-  // step before the quad's (half's) end, so that the last step can read the
+  // One quad of ng groups (constants, as is everything but q; par: its parity;
+  // first: known to be quad 0, behind which there is no bias term to add: in the
+  // rolled loop quad 0 adds zeros): steps s = gi * N + n, the step registers
+  // alternating by s.  Two steps before the end of each half, when the last of its
+  // codes are read, the next half's go from registers to the wave's own LDS and the
+  // loads of the same half R quads on are issued into the registers (ng_next,
+  // ng_second, ng_load: groups of quads q + 1, q + R and q + 1 + R, 0: none).  The A
+  // rows of the next quad go along with M <= 2, else half a quad ahead.  The barrier
+  // is one step before the quad's (half's) end, so that the last step can read the
   // next fragments.
-  auto quad = [&](int q, int par, int ng, int ng_next, int ng_second, int ng_load) {
+  auto quad = [&](int q, int par, int ng, int ng_next, int ng_second, int ng_load, bool first) {
     const int ns = ng * N, rs = (par + 1) % R;
-#pragma unroll
-    for (int st = 0; st < 4 * N; ++st) {
-      if (st >= ns) continue;
-      const int gi = st / N, n = st % N, j = n % NPROJ, cb = n / NPROJ;
+    // the next chunk's scales and biases: the LDS of a chunk's scales is free from
+    // its quad 3 on, of its biases from that quad's second group on
+    const bool chunk = q / 4 + 1 < I::NCH;
+    if ((q & 3) == 2 && chunk) load_s(q / 4 + 1, s0, s1, sv);
+    if ((q & 3) == 3 && chunk) {
+      store_s(0, sv);
+      load_s(q / 4 + 1, o0, o1, sv);
+    }
+    if (!QA && ng > 2) load_a(q, 2, ng, 0);
+    // a step; G0: of the quad's first group
+    auto step = [&](int st, auto G0) {
+      constexpr bool g0 = decltype(G0)::value;
+      const int gi = g0 ? 0 : st / N, n = st % N, j = n % NPROJ, cb = n / NPROJ;
       const int cur = st & 1, prv = cur ^ 1;
       // the block folded here: the step before's
       const int pn = (n + N - 1) % N, pj = pn % NPROJ, pcb = pn / NPROJ;
       const bool dec = st + 1 < ns || ng_next > 0;   // there is a step after
       const bool last = st + 1 == ns;
       const bool half_end = last || (!QA && st == 2 * N - 1);
+      // the bias term of the quad before, block n; added in the step after where
+      // there are registers to hold it
+      const bool bias = g0 && !first, pend = BZ == M && !first && st > 0 && st <= N;
+      if (last && (q & 3) == 3 && chunk) store_s(1, sv);
       const int nbuf = QA ? par ^ 1 : last ? 0 : 1;   // the A buffer after this one
-      if (!QA && st == 0 && ng > 2) load_a(q, 2, ng, 0);
       if (!QA && st == (ng > 2 ? 2 * N : 0) && ng_next > 0) load_a(q + 1, 0, ng_next, 0);
       if (!QA && half_end && (!last || ng_next > 0))
         store_a(nbuf, last ? 0 : 2, last ? ng_next : ng, 0);
@@ -676,12 +688,13 @@ __device__ __forceinline__ void grouped_item(
       const bool nxa = n == N - 1 && dec;
       const int ag = half_end ? nbuf * AG : QA ? par * AG + gi + 1 : gi + 1;
       const uint4 *an = L.a + ag * (AROWS * 8);
-      const uint32_t h = gi < 2 ? scur[n].x : scur[n].y;
+      const uint2 scur_q = scur[n];
+      const uint32_t h = gi < 2 ? scur_q.x : scur_q.y;
       S[cur] = __uint_as_float((gi & 1) ? (h & 0xffff0000u) : (h << 16));
       if (last && ng_next > 0)
 #pragma unroll
         for (int i = 0; i < N; ++i)
-          scur[i] = *reinterpret_cast<const uint2 *>(sl + (i * 16 + col) * SPB + (q + 1) * 8);
+          scur[i] = read_s(0, q + 1, i);
       const uint4 fb0 = make_uint4(bf[cur][0], bf[cur][1], bf[cur][2], bf[cur][3]);
       const uint4 fb1 = make_uint4(bf[cur][4], bf[cur][5], bf[cur][6], bf[cur][7]);
       uint2 cw = creg[prv];
@@ -690,6 +703,7 @@ __device__ __forceinline__ void grouped_item(
 #pragma unroll
       for (int rb = 0; rb < M; ++rb) {
         f32x4_t &o = acc[rb][pcb][pj];
+        if (pend) add_block(o, bz[rb % BZ]);
 #pragma unroll
         for (int e = 0; e < 4; ++e) o[e] += S[prv] * c[rb][e];
         pin(o);
@@ -700,6 +714,10 @@ __device__ __forceinline__ void grouped_item(
       }
 #pragma unroll
       for (int rb = 0; rb < M; ++rb) {
+        if constexpr (g0) if (bias) {
+          bz[rb % BZ] = bias_block(rb, n);
+          pin(bz[rb % BZ]);
+        }
         c[rb] = mfma16x16x32(a1[rb], fb1, c[rb]);
         pin(c[rb]);
         if (nxa) a1[rb] = an[rb * 128 + ard[1]];
@@ -707,32 +725,63 @@ __device__ __forceinline__ void grouped_item(
 #pragma unroll
           for (int m = 8 * rb / M; m < 8 * (rb + 1) / M; ++m)
             bf[prv][m] = decode(cw, m), pin(bf[prv][m]);
+        if constexpr (g0) if (bias && BZ < M) add_block(acc[rb][cb][j], bz[0]);
         __builtin_amdgcn_sched_barrier(0);
       }
-    }
+      if constexpr (g0) {   // this quad's factors
+        C[n] = fmaf(-128.f, pick(scur_q), pick(bnx));
+        if (n + 1 < N) bnx = read_s(1, q, n + 1);
+      }
+      if (last) {
+        if (ng_next > 0) bnx = read_s(1, q + 1, 0);
+#pragma unroll
+        for (int rb = 0; rb < M; ++rb) ra[rb] = rsl[rb * 16 * I::RSP + 4 * q];
+      }
+    };
+    // (two loops, each small enough to be unrolled)
+#pragma unroll
+    for (int st = 0; st < N; ++st) step(st, std::true_type());
+#pragma unroll
+    for (int st = N; st < 4 * N; ++st)
+      if (st < ns) step(st, std::false_type());
   };
   // the quads whose loads are whole quads (in pairs where the registers
   // alternate), then the rest
   constexpr int QR = R == 2 || QA ? 2 : 1, QP = NQ > R + 2 ? (NQ - R - 2) / QR * QR : 0;
 #pragma unroll 1
   for (int q = 0; q < QP; q += QR) {
-    quad(q, 0, 4, 4, 4, 4);
-    if (QR == 2) quad(q + 1, 1, 4, 4, 4, 4);
+    quad(q, 0, 4, 4, 4, 4, false);
+    if (QR == 2) quad(q + 1, 1, 4, 4, 4, 4, false);
   }
 #pragma unroll
   for (int q = QP; q < NQ; ++q) {
     auto groups = [](int i) { return i < NQ - 1 ? 4 : i == NQ - 1 ? NGL : 0; };
-    quad(q, q & 1, groups(q), groups(q + 1), groups(q + R), groups(q + 1 + R));
+    quad(q, q & 1, groups(q), groups(q + 1), groups(q + R), groups(q + 1 + R), q == 0);
   }
-  {   // the last step's fold
-    constexpr int last = (NGL * N - 1) & 1;
+  {   // the last step's fold and the last quad's bias term
+    constexpr int last = (NGL * N - 1) & 1, lc = (N - 1) / NPROJ, lj = (N - 1) % NPROJ;
+#pragma unroll
+    for (int rb = 0; rb < M; ++rb) {
+      if (NGL == 1 && NQ > 1 && BZ == M) add_block(acc[rb][lc][lj], bz[rb % BZ]);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) acc[rb][lc][lj][e] += S[last] * c[rb][e];
+    }
 #pragma unroll
     for (int rb = 0; rb < M; ++rb)
 #pragma unroll
-      for (int e = 0; e < 4; ++e)
-        acc[rb][(N - 1) / NPROJ][(N - 1) % NPROJ][e] += S[last] * c[rb][e];
+      for (int n = 0; n < N; ++n) {
+        const f32x4_t b = bias_block(rb, n);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc[rb][n / NPROJ][n % NPROJ][e] += b[e];
+      }
   }
 
+  int tid_e = tid;
+  pin(tid_e);
+  float pb[CB][NPROJ];
+#pragma unroll
+  for (int n = 0; n < N; ++n)
+    pb[n / NPROJ][n % NPROJ] = PBIAS ? L.pb[wave * 64 + n * 16 + (tid_e & 15)] : 0.f;
   if (GU) {
     // the activations go through LDS (the A buffers, free once every wave is
     // past the last quad) and out as whole rows, 16 bytes per lane, in x_pairs
@@ -753,25 +802,23 @@ __device__ __forceinline__ void grouped_item(
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
           const int rr = rb * 16 + 4 * kq + e;
-          const float hv = apply_act(act, acc[rb][cb][0][e] + pb[0][cb],
-                                     acc[rb][cb][NPROJ - 1][e] + pb[NPROJ - 1][cb], alpha, limit);
+          const float hv = apply_act(act, acc[rb][cb][0][e] + pb[cb][0],
+                                     acc[rb][cb][NPROJ - 1][e] + pb[cb][NPROJ - 1], alpha, limit);
           tile[rr * NB + (npl ^ swz(rr))] = (uint16_t)f32_to_bf16(hv);
         }
     }
     __syncthreads();
     constexpr int CPR = NB / 8;                       // 16-byte pieces per row
 #pragma unroll 1
-    for (int i = tid; i < ROWS * CPR; i += kMmThreads) {
+    for (int it = 0; it < (ROWS * CPR + kMmThreads - 1) / kMmThreads; ++it) {
+      const int i = tid_e + kMmThreads * it;
+      if (i >= ROWS * CPR) break;   // (whole waves)
       const int r = i / CPR, c = i % CPR, f = nb0 + c * 8;
       const uint4 v = *reinterpret_cast<const uint4 *>(tile + r * NB + ((c * 8) ^ swz(r)));
-      const uint32_t in[4] = {v.x, v.y, v.z, v.w};
-      float sm = 0.f;
-#pragma unroll
-      for (int m = 0; m < 4; ++m) sm += bf16_to_f32(in[m] & 0xffffu) + bf16_to_f32(in[m] >> 16);
-      sm = group_sum<8>(sm);
+      const float sm = h_row_sum<F>(v);
       if (r < rows && f < F) {
         *reinterpret_cast<uint4 *>(h_out + (int64_t)(r0 + r) * F + f) = v;
-        put_row_sum(rs_out + (int64_t)(r0 + r) * (3 * rs_pitch(F)), rs_pitch(F), f / 64, c & 7, sm);
+        if ((c & 7) == 0) rs_out[(int64_t)(r0 + r) * rs_pitch(F) + f / 64] = sm;
       }
     }
   } else {
@@ -793,11 +840,12 @@ __device__ __forceinline__ void grouped_item(
 #pragma unroll
           for (int cb = 0; cb < CB; ++cb)
             tile[(rr - r2 * 16) * NB + (((wave * CB + cb) * 16 + col) ^ (kq << 4))] =
-                sc * (acc[rb][cb][0][e] + pb[0][cb]);
+                sc * (acc[rb][cb][0][e] + pb[cb][0]);
         }
       __syncthreads();
 #pragma unroll 4
-      for (int i = tid; i < 32 * CPR; i += kMmThreads) {
+      for (int it = 0; it < 32 * CPR / kMmThreads; ++it) {
+        const int i = tid_e + kMmThreads * it;
         const int r = i / CPR, cc = (i % CPR) * 4, rr = r2 * 16 + r;
         if (rr < rows && (D % NB == 0 || nb0 + cc < D))
           *reinterpret_cast<uint4 *>(yp + (int64_t)L.rperm[rr] * D + nb0 + cc) =
@@ -816,8 +864,8 @@ constexpr int kXcdTiles = 64;
 
 template <int CB, int D, int F, bool PBIAS, bool GU>
 __device__ __forceinline__ void grouped_items(
-    const PoolArgs &pa, const uint16_t *aq, const uint16_t *ars, TokenOf tok,
-    const int32_t *perm, const int4 *tiles, int n_tiles, int4 first, uint16_t *h_out, uint16_t *rs_out,
+    const PoolArgs &pa, const uint16_t *aq, const float *ars, TokenOf tok,
+    const int32_t *perm, const int4 *tiles, int n_tiles, int4 first, uint16_t *h_out, float *rs_out,
     const float *scores, float *yp, int act, float alpha, float limit, const GLds &L) {
   constexpr int NOUT = GU ? F : D, NB = 16 * CB * kMmWaves, NBK = (NOUT + NB - 1) / NB;
   constexpr int NP = PBIAS ? 4 : 3, NPROJ = GU ? 2 : 1;
@@ -857,10 +905,10 @@ __device__ __forceinline__ void grouped_items(
 // kWideItems such items, CBN otherwise
 template <int D, int F, bool PBIAS, int CBW, int CBN, bool GU>
 __global__ __launch_bounds__(kMmThreads) __attribute__((amdgpu_waves_per_eu(2))) void
-grouped_mm_kernel(PoolArgs pa, const uint16_t *__restrict__ aq, const uint16_t *__restrict__ ars,
+grouped_mm_kernel(PoolArgs pa, const uint16_t *__restrict__ aq, const float *__restrict__ ars,
                   TokenOf tok, const int32_t *__restrict__ perm,
                   const int4 *__restrict__ tiles, const int32_t *__restrict__ n_tiles,
-                  uint16_t *__restrict__ h_out, uint16_t *__restrict__ rs_out,
+                  uint16_t *__restrict__ h_out, float *__restrict__ rs_out,
                   const float *__restrict__ scores, float *__restrict__ yp, int act, float alpha,
                   float limit) {
   constexpr int NOUT = GU ? F : D, NBW = 16 * CBW * kMmWaves;
@@ -868,11 +916,13 @@ grouped_mm_kernel(PoolArgs pa, const uint16_t *__restrict__ aq, const uint16_t *
   __shared__ uint4 a_l[4 * kTileM * 8];
   static_assert(NW <= 4, "code region");
   __shared__ uint4 b_l[kMmWaves * kCodeBytes / 16];
-  // (a fragment read of the last row may run past it)
-  __shared__ uint4 s_l[kMmWaves * NW * GDim<GU ? D : F>::SPB + 1];
+  __shared__ uint4 s_l[kMmWaves * NW * 64];
+  __shared__ uint4 rs_l[kTileM * GDim<GU ? D : F>::RSP / 4];
+  __shared__ float pb_l[PBIAS ? kMmThreads : 1];
   __shared__ int rp_l[GU ? 1 : kTileM];
   __shared__ float rc_l[GU ? 1 : kTileM];
-  const GLds L{a_l, reinterpret_cast<char *>(b_l), reinterpret_cast<char *>(s_l), rp_l, rc_l};
+  const GLds L{a_l, reinterpret_cast<char *>(b_l), reinterpret_cast<char *>(s_l),
+               reinterpret_cast<float *>(rs_l), pb_l, rp_l, rc_l};
   // a few tiles' items (narrow, dealt in order): the first one's tile is loaded
   // beside the tile count, not after it (past the count it is not used; the
   // workspace goes on past the tile list)
@@ -914,8 +964,8 @@ __global__ __launch_bounds__(256) void combine_pairs_kernel(
 // ---------------------------------------------------------------------------
 template <int D, int F, bool PB, int CBW, int CBN>
 static void launch_gg(dim3 g, hipStream_t s, const PoolArgs &pa, const uint16_t *xq,
-                      const uint16_t *rsx, int k, const int32_t *perm, const int4 *tiles,
-                      const int32_t *nt, uint16_t *h, uint16_t *rsh, int act, float alpha,
+                      const float *rsx, int k, const int32_t *perm, const int4 *tiles,
+                      const int32_t *nt, uint16_t *h, float *rsh, int act, float alpha,
                       float limit) {
   hipLaunchKernelGGL((grouped_mm_kernel<D, F, PB, CBW, CBN, true>), g, dim3(kMmThreads), 0, s, pa,
                      xq, rsx, token_of(k), perm, tiles, nt, h, rsh, nullptr, nullptr, act, alpha,
@@ -923,7 +973,7 @@ static void launch_gg(dim3 g, hipStream_t s, const PoolArgs &pa, const uint16_t 
 }
 template <int D, int F, bool PB, int CBW, int CBN>
 static void launch_gd(dim3 g, hipStream_t s, const PoolArgs &pa, const uint16_t *hq,
-                      const uint16_t *rsh, const float *sc, const int32_t *perm,
+                      const float *rsh, const float *sc, const int32_t *perm,
                       const int4 *tiles, const int32_t *nt, float *yp) {
   hipLaunchKernelGGL((grouped_mm_kernel<D, F, PB, CBW, CBN, false>), g, dim3(kMmThreads), 0, s,
                      pa, hq, rsh, token_of(1), perm, tiles, nt, nullptr, nullptr, sc, yp, 0, 0.f, 0.f);
@@ -958,22 +1008,22 @@ GroupedWs grouped_ws(int64_t T, int k, int D, int F) {
   w.off_ntiles = o; o += al(4);
   w.off_yp = o; o += al((size_t)P * D * 4);
   w.off_xq = o; o += al((size_t)T * D * 2);
-  w.off_rsx = o; o += al((size_t)T * 3 * rs_pitch(D) * 2);
+  w.off_rsx = o; o += al((size_t)T * rs_pitch(D) * 4);
   w.off_hq = o; o += al((size_t)P * F * 2);
-  w.off_rsh = o; o += al((size_t)P * 3 * rs_pitch(F) * 2);
+  w.off_rsh = o; o += al((size_t)P * rs_pitch(F) * 4);
   w.total = o;
   return w;
 }
 
 // (in launches of at most 2^30 pieces, so the kernel's indices fit 32 bits)
-static void launch_prep(const uint16_t *src, int64_t rows, int K, uint16_t *dst, uint16_t *rs,
+static void launch_prep(const uint16_t *src, int64_t rows, int K, uint16_t *dst, float *rs,
                         hipStream_t s) {
   const int64_t chunk = ((int64_t)1 << 30) / (K / 8);
   for (int64_t r0 = 0; r0 < rows; r0 += chunk) {
     const int64_t nr = std::min(chunk, rows - r0);
     const int64_t n = nr * (K / 8);
     hipLaunchKernelGGL(grouped_prep_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s,
-                       src + r0 * K, nr, K, dst + r0 * K, rs + r0 * 3 * rs_pitch(K));
+                       src + r0 * K, nr, K, dst + r0 * K, rs + r0 * rs_pitch(K));
   }
 }
 
@@ -988,9 +1038,9 @@ void launch_grouped(const GroupedLaunch *G, const PoolArgs &pa, const int32_t *r
   int32_t *ntiles = reinterpret_cast<int32_t *>(ws + w.off_ntiles);
   float *yp = reinterpret_cast<float *>(ws + w.off_yp);
   uint16_t *xq = reinterpret_cast<uint16_t *>(ws + w.off_xq);
-  uint16_t *rsx = reinterpret_cast<uint16_t *>(ws + w.off_rsx);
+  float *rsx = reinterpret_cast<float *>(ws + w.off_rsx);
   uint16_t *hq = reinterpret_cast<uint16_t *>(ws + w.off_hq);
-  uint16_t *rsh = reinterpret_cast<uint16_t *>(ws + w.off_rsh);
+  float *rsh = reinterpret_cast<float *>(ws + w.off_rsh);
   const int nkeys = pa.n_slots + pa.n_records;
   const int64_t xpieces = (int64_t)T * (D / 8);
   if (xpieces < ((int64_t)1 << 30)) {   // grouping and x prep in one launch

@@ -73,10 +73,10 @@ constexpr int kGroupedMaxWGs = 2048;    // grid cap; workgroups loop over items
 struct GroupedLaunch {
   int d_model, d_ff, has_bias;
   int nb_up, nb_down;   // fewest output features per work item of gate/up and of down
-  void (*gate_up)(dim3, hipStream_t, const PoolArgs &, const uint16_t *, const uint16_t *, int,
-                  const int32_t *, const int4 *, const int32_t *, uint16_t *, uint16_t *, int,
+  void (*gate_up)(dim3, hipStream_t, const PoolArgs &, const uint16_t *, const float *, int,
+                  const int32_t *, const int4 *, const int32_t *, uint16_t *, float *, int,
                   float, float);
-  void (*down)(dim3, hipStream_t, const PoolArgs &, const uint16_t *, const uint16_t *,
+  void (*down)(dim3, hipStream_t, const PoolArgs &, const uint16_t *, const float *,
                const float *, const int32_t *, const int4 *, const int32_t *, float *);
 };
 struct GroupedWs {

@@ -416,11 +416,11 @@ def _plain_records(geom, n, parts):
 def test_grouped_activation_far_gates(act):
     """Gates far outside the sigmoid's range give what the activation's formula
     and the decode kernels give: zero far below, the gate (or its limit) far
-    above.  Expert e has gate value g[e] and up value u in one feature and zeros
-    elsewhere, and passes it on: with x = 1/256 the gate is its quant bias times
+    above, NaN for minus infinity.  Expert e has gate value g[e] and up value u in
+    one feature and zeros elsewhere, and passes it on: with x = 1/256 the gate is its quant bias times
     the sum of x, which is 1."""
     geom = G.SMALL.with_(act=act)
-    g = [-3.3e38, -1e30, -1e8, -1e5, -1000.0, -104.0, -89.0, -80.0,
+    g = [-3.3e38, -1e30, -1e8, -float("inf"), -1000.0, -104.0, -89.0, -80.0,
          -20.0, -3.0, 0.0, 5.0, 30.0, 100.0, 1e8, 1e30]
     g = torch.tensor(g, dtype=torch.bfloat16, device="cuda")
     assert g.numel() == geom.n_experts
@@ -450,10 +450,55 @@ def test_grouped_activation_far_gates(act):
     else:
         v = v.clamp(max=geom.limit)
         want = v * torch.sigmoid(geom.alpha * v) * (u + 1)
+    want[g == -float("inf")] = float("nan")
     for got in (y, yd):
         got = got[:, :1].double().squeeze(1)
+        assert torch.equal(got.isnan(), want.isnan()), got
         # h is bf16, 8 significant bits: 2^-8 of its value at most, and fp32's
         # exp; below -88.7 that is infinite and h zero, where the true value is
         # under 89 e^-88.7 (u + 1)
         ok = (got - want).abs() <= want.abs() * (2.0 ** -8 + 1e-5) + 1.1e-36
-        assert bool(ok.all()), torch.stack([got, want])
+        assert bool((ok | want.isnan()).all()), torch.stack([got, want])
+
+
+@pytest.mark.parametrize("geom", [G.QWEN3_30B_A3B, G.GPT_OSS_120B, G.SMALL],
+                         ids=["qwen3", "gptoss", "small"])
+def test_grouped_offset_cancels_within_four_groups(geom):
+    """The codes go into the products as 128 + q; the offset is taken out again
+    every 4 groups, before the sum is carried on, so rows of one sign lose nothing.
+    With h whole numbers below 256 (of a unit) and one power of two as every scale, the
+    sum of a group is below 64 * 255 * 143, of four groups below 9.4e6, and the part
+    carried on, sum of h (q - 8), below 64 * 45 * 255 * 8 = 5.9e6: all of them and
+    their sums are whole and below 2^24, exact in fp32 in any order within the four
+    groups.  (Offsets taken out after all 45 groups: 9.4e7, rounded to 8.)"""
+    geom = geom.with_(act=_lib.MOE_ACT_SWIGLU)
+    D, F, E = geom.d_model, geom.d_ff, 5
+    gen = synth.generator("cuda", 20260081)
+    up = torch.randint(128, 256, (E, F, 1), generator=gen, device="cuda") / 128.0
+    codes = torch.randint(-2 ** 31, 2 ** 31, (E, D, F // 8), generator=gen, device="cuda")
+    step = 2.0 ** -6
+    rec = _plain_records(geom, E, {
+        "gate_proj.biases": torch.tensor(32.0, device="cuda"), "up_proj.biases": up,
+        "down_proj.weight": codes, "down_proj.scales": torch.tensor(step, device="cuda"),
+        "down_proj.biases": torch.tensor(-8 * step, device="cuda")})
+    pool = SlotPool(geom, 1, "cuda", store=rec)
+    # tiles of 64 + 16, 32, 48, 5 and 1 rows
+    ids = torch.repeat_interleave(torch.arange(E), torch.tensor([80, 32, 48, 5, 1])).cuda()
+    T = ids.numel()
+    # x sums to a power of two p in every row: gate 32 p (past where silu is the
+    # identity in fp32), up p * up, h 32 p^2 up, exact in bf16
+    n_in = 1 << (D.bit_length() - 1)
+    p = 2.0 ** (torch.arange(T, device="cuda") % 4)
+    x = torch.zeros((T, D), dtype=torch.bfloat16, device="cuda")
+    x[:, :n_in] = (p / n_in)[:, None].to(torch.bfloat16)
+    y = torch.empty((T, D), device="cuda")
+    ops.ffn_grouped(pool, (-1 - ids).to(torch.int32).view(T, 1).contiguous(),
+                    torch.ones((T, 1), device="cuda"), x, out_f32=y)
+    torch.cuda.synchronize()
+    ops.check_device_error()
+    nib = torch.arange(8, device="cuda")
+    for e in range(E):
+        q = ((codes[e][:, :, None] >> (4 * nib)) & 15).reshape(D, F).double() - 8
+        want = step * (q * (32 * up[e, :, 0].double())).sum(1)
+        t = ids == e
+        assert torch.equal(y[t].double(), p[t, None].double() ** 2 * want), e
