@@ -371,33 +371,53 @@ def test_multi_token_stack_graph_replays_equal_eager(T, block, expect):
     torch.cuda.empty_cache()
 
 
-@pytest.mark.parametrize("geom,T", [(G.QWEN3_30B_A3B, 2560), (G.GPT_OSS_120B, 1024)],
+@pytest.mark.parametrize("geom,T", [(G.QWEN3_30B_A3B, 2560), (G.GPT_OSS_120B, 2048)],
                          ids=["qwen3", "gptoss"])
 def test_grouped_wide_items_equal_narrow_items(geom, T):
-    """A call of enough tiles for the wide work items (2,048 of them: 128 of
-    Qwen3's gate/up features or 256 outputs each) gives the rows of calls that
-    take the narrow ones, bit for bit: tiles of 1 to 64 rows, the last feature
-    block of gpt-oss partly past the matrix."""
+    """A call of enough tiles for the wide work items of both kernels (2,048 of
+    them, of 128 gate/up features and of 256 outputs) gives the rows of calls that
+    take the narrow ones, bit for bit: tiles of 1 to 64 rows, the last feature block
+    of gpt-oss partly past the matrix in both.  The rows of tokens whose experts all
+    have full 64-row tiles are checked against the fp64 oracle too."""
+    wide_items = 2048
     layer = Layer(geom, geom.n_experts + 8, seed=20260071, router_bias=True)
     rng = np.random.default_rng(20260072)
-    # experts of every row-block count: popularity from 1 to 200 rows a tile list
+    # experts of every row-block count
     p = np.linspace(0.05, 1.0, geom.n_experts)
     z = np.log(p) + rng.gumbel(size=(T, geom.n_experts))
     ids = np.argpartition(-z, geom.top_k - 1, axis=1)[:, :geom.top_k]
-    n_tiles = sum(-(-c // 64) for c in np.bincount(ids.ravel(), minlength=geom.n_experts))
-    assert n_tiles * (-(-geom.d_ff // 128)) >= 2048
+
+    def items(rows):   # work items of each kernel as wide ones
+        c = np.bincount(rows.ravel(), minlength=geom.n_experts)
+        n_tiles = (-(-c // 64)).sum()
+        return n_tiles * (-(-geom.d_ff // 128)), n_tiles * (-(-geom.d_model // 256))
+
+    assert min(items(ids)) >= wide_items
     refs = layer.table[torch.tensor(ids, device="cuda")].to(torch.int32).contiguous()
-    scores = torch.tensor(rng.dirichlet(np.ones(geom.top_k), T).astype(np.float32), device="cuda")
+    sc = rng.dirichlet(np.ones(geom.top_k), T).astype(np.float32)
+    scores = torch.tensor(sc, device="cuda")
     x = bf16_randn((T, geom.d_model), seed=20260073)
     y = torch.zeros((T, geom.d_model), dtype=torch.float32, device="cuda")
     ops.ffn_grouped(layer.pool, refs, scores, x, out_f32=y)
-    for n in (7, 97):
-        yn = torch.zeros((n, geom.d_model), dtype=torch.float32, device="cuda")
-        ops.ffn_grouped(layer.pool, refs[:n].contiguous(), scores[:n].contiguous(),
-                        x[:n].contiguous(), out_f32=yn)
+    step = 256 if geom.d_ff < 2048 else 24   # few enough tiles for narrow items
+    for a, b in [(0, 7)] + [(a, min(a + step, T)) for a in range(0, T, step)]:
+        assert max(items(ids[a:b])) < wide_items
+        yn = torch.zeros((b - a, geom.d_model), dtype=torch.float32, device="cuda")
+        ops.ffn_grouped(layer.pool, refs[a:b].contiguous(), scores[a:b].contiguous(),
+                        x[a:b].contiguous(), out_f32=yn)
         torch.cuda.synchronize()
         ops.check_device_error()
-        assert torch.equal(yn, y[:n]), n
+        assert torch.equal(yn, y[a:b]), (a, b)
+    counts = np.bincount(ids.ravel(), minlength=geom.n_experts)
+    full = np.nonzero((counts[ids] >= 64).all(axis=1))[0][-6:]
+    y64 = N.moe_block_batch(bf16_values(x)[full], ids[full], sc[full].astype(np.float64),
+                            layer.expert, "gptoss" if geom.has_proj_bias else "qwen3", "f64",
+                            geom.alpha, geom.limit)
+    o32 = y.cpu().numpy()
+    err = max(N.rel_err(o32[t], y64[i]) for i, t in enumerate(full))
+    assert err < TOL, err
+    del layer
+    torch.cuda.empty_cache()
 
 
 def _plain_records(geom, n, parts):
