@@ -858,9 +858,12 @@ __device__ __forceinline__ void grouped_item(
 // Items of a call: (tile, feature block).  From kXcdTiles tiles on the items
 // of one tile go to workgroups of one XCD (workgroup i runs on XCD i % 8), so
 // the tile's rows are read from HBM once and from that XCD's L2 by the other
-// items, and a hot expert's codes once per XCD.  With fewer tiles that would
-// leave XCDs idle; the items are dealt in order.
-constexpr int kXcdTiles = 64;
+// items, and a hot expert's codes once per XCD.  With fewer tiles that leaves some
+// XCDs with a tile more than others; the items are dealt in order.  A block by XCD
+// from 64 tiles on / from 128 / never: Qwen3 32 tokens (75 tiles) 70.2 / 69.1 / 68.4
+// us, 64 tokens (99) 85.8 / 83.8 / 83.7, gpt-oss 60 tokens (73) 252 / 245 / 248;
+// Qwen3 2,048 tokens (319) 354 / 350 / 358, 4,096 tokens (572) 622 / 626 / 640.
+constexpr int kXcdTiles = 128;
 
 template <int CB, int D, int F, bool PBIAS, bool GU>
 __device__ __forceinline__ void grouped_items(
