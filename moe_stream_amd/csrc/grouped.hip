@@ -868,7 +868,7 @@ constexpr int kXcdTiles = 128;
 template <int CB, int D, int F, bool PBIAS, bool GU>
 __device__ __forceinline__ void grouped_items(
     const PoolArgs &pa, const uint16_t *aq, const float *ars, TokenOf tok,
-    const int32_t *perm, const int4 *tiles, int n_tiles, int4 first, uint16_t *h_out, float *rs_out,
+    const int32_t *perm, const int4 *tiles, int n_tiles, uint16_t *h_out, float *rs_out,
     const float *scores, float *yp, int act, float alpha, float limit, const GLds &L) {
   constexpr int NOUT = GU ? F : D, NB = 16 * CB * kMmWaves, NBK = (NOUT + NB - 1) / NB;
   constexpr int NP = PBIAS ? 4 : 3, NPROJ = GU ? 2 : 1;
@@ -879,7 +879,7 @@ __device__ __forceinline__ void grouped_items(
     const int tile = by_xcd ? (j / NBK) * 8 + (item & 7) : item / NBK;
     const int nb0 = (by_xcd ? j % NBK : item % NBK) * NB;
     if (tile >= n_tiles) continue;
-    const int4 tl = first.z && item == (int)blockIdx.x && !by_xcd ? first : tiles[tile];
+    const int4 tl = tiles[tile];
     const int ref = tl.x, r0 = tl.y, rows = tl.z;
     bool bad = false;
 #pragma unroll
@@ -926,18 +926,12 @@ grouped_mm_kernel(PoolArgs pa, const uint16_t *__restrict__ aq, const float *__r
   __shared__ float rc_l[GU ? 1 : kTileM];
   const GLds L{a_l, reinterpret_cast<char *>(b_l), reinterpret_cast<char *>(s_l),
                reinterpret_cast<float *>(rs_l), pb_l, rp_l, rc_l};
-  // a few tiles' items (narrow, dealt in order): the first one's tile is loaded
-  // beside the tile count, not after it (past the count it is not used; the
-  // workspace goes on past the tile list)
-  constexpr int NBKN = (NOUT + 16 * CBN * kMmWaves - 1) / (16 * CBN * kMmWaves);
-  int4 first = tiles[blockIdx.x / NBKN];
-  int nt = *n_tiles;
-  asm volatile("" : "+s"(nt), "+s"(first.x), "+s"(first.y), "+s"(first.z));
+  const int nt = *n_tiles;
   if (nt * ((NOUT + NBW - 1) / NBW) >= kWideItems)
-    grouped_items<CBW, D, F, PBIAS, GU>(pa, aq, ars, tok, perm, tiles, nt, make_int4(0, 0, 0, 0), h_out, rs_out,
+    grouped_items<CBW, D, F, PBIAS, GU>(pa, aq, ars, tok, perm, tiles, nt, h_out, rs_out,
                                         scores, yp, act, alpha, limit, L);
   else
-    grouped_items<CBN, D, F, PBIAS, GU>(pa, aq, ars, tok, perm, tiles, nt, first, h_out, rs_out,
+    grouped_items<CBN, D, F, PBIAS, GU>(pa, aq, ars, tok, perm, tiles, nt, h_out, rs_out,
                                         scores, yp, act, alpha, limit, L);
 }
 
