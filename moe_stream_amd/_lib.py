@@ -163,5 +163,6 @@ def check(rc: int) -> int:
 
 
 def stream_ptr(stream=None) -> int:
-    s = stream if stream is not None else torch.cuda.current_stream()
-    return int(s.cuda_stream)
+    if stream is None:   # the current stream's handle, without a stream object
+        return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
+    return int(stream.cuda_stream)

@@ -6,6 +6,8 @@ host, then launches on the current stream (or `stream`).
 from __future__ import annotations
 
 import ctypes as C
+import threading
+from collections import OrderedDict
 
 import torch
 
@@ -30,21 +32,65 @@ def _req(t, dtype, name, numel=None, device=None):
         raise ValueError(f"{name}: on {t.device}, expected {device}")
 
 
-class Workspace:
-    """Grow-only device scratch buffers, one per purpose and device."""
+def _side(stream, device):
+    """`stream` as a torch stream where it is another than the current one (any
+    object with a cuda_stream handle), else None."""
+    if stream is None or stream.cuda_stream == torch.cuda.current_stream(device).cuda_stream:
+        return None
+    if isinstance(stream, torch.cuda.Stream):
+        return stream
+    return torch.cuda.ExternalStream(int(stream.cuda_stream), device=device)
+
+
+def _empty(shape, dtype, device, side):
+    """A tensor for kernels on stream `side` (None: the current one) to write:
+    allocated in that stream's order, so that the work of the block's last owner is
+    not still under way, and kept from reuse while the current stream reads it."""
+    if side is None:
+        return torch.empty(shape, dtype=dtype, device=device)
+    cur = torch.cuda.current_stream(device)
+    with torch.cuda.stream(side):
+        t = torch.empty(shape, dtype=dtype, device=device)
+    t.record_stream(cur)
+    return t
+
+
+class Workspace(threading.local):
+    """Grow-only device scratch buffers, one per purpose, device and stream in every
+    thread: a call's launches are not one unit, so calls that can run beside each
+    other must not share one.  A buffer belongs to its stream's order (a replaced or
+    evicted one is reused only behind the calls that hold it).  The KEEP used last
+    stay; a call under graph capture takes a buffer of the graph's own instead, since
+    a replay can run beside any stream's calls."""
+
+    KEEP = 16
 
     def __init__(self):
-        self._bufs = {}
+        self._bufs = OrderedDict()
 
-    def get(self, key, nbytes: int, device, zero: bool = False) -> torch.Tensor:
-        k = (key, str(device))
+    def get(self, key, nbytes: int, device, handle: int = 0, zero: bool = False,
+            side=None) -> torch.Tensor:
+        """At least nbytes for calls on the stream of that handle: `side`, or the
+        current one."""
+        if side is not None:
+            with torch.cuda.stream(side):
+                return self.get(key, nbytes, device, handle, zero)
+        k = (key, device, handle)
         b = self._bufs.get(k)
-        if b is None or b.numel() < nbytes:
-            b = torch.zeros(max(nbytes, 256), dtype=torch.uint8, device=device)
+        own = device.type == "cuda" and _capturing()
+        if b is None or own or b.numel() < nbytes:
+            b = (torch.zeros if zero else torch.empty)(max(nbytes, 256), dtype=torch.uint8,
+                                                       device=device)
+            if own:
+                return b
             self._bufs[k] = b
+            if len(self._bufs) > self.KEEP:
+                self._bufs.popitem(last=False)
+        self._bufs.move_to_end(k)
         return b
 
 
+_capturing = torch.cuda.is_current_stream_capturing
 _WS = Workspace()
 
 
@@ -80,7 +126,7 @@ def ffn_decode_up(pool, slot_refs: torch.Tensor, x: torch.Tensor,
     if need == 0:
         raise ValueError(f"moe_ffn_decode_up: unsupported T={T}, k={k}")
     if workspace is None:
-        workspace = torch.empty(need, dtype=torch.uint8, device=x.device)
+        workspace = _empty(need, torch.uint8, x.device, _side(stream, x.device))
     _lib.check(L.moe_ffn_decode_up(
         C.byref(pool.c_view()), C.byref(g), _p(slot_refs), _p(x), T, k,
         _p(workspace), workspace.numel(), _lib.stream_ptr(stream)))
@@ -100,7 +146,8 @@ def ffn_decode_down(pool, slot_refs: torch.Tensor, scores: torch.Tensor,
     _req(scores, torch.float32, "scores", T * k, pool.device)
     _req(workspace, torch.uint8, "workspace", device=pool.device)
     if out is None and out_f32 is None:
-        out = torch.empty((T, D), dtype=torch.bfloat16, device=slot_refs.device)
+        dev = slot_refs.device
+        out = _empty((T, D), torch.bfloat16, dev, _side(stream, dev))
     if out is not None:
         _req(out, torch.bfloat16, "out", T * D, pool.device)
     if out_f32 is not None:
@@ -123,7 +170,7 @@ def slot_lookup(table: torch.Tensor, ids: torch.Tensor,
     _req(ids, torch.int32, "ids", device=table.device)
     if miss is not None:
         _req(miss, torch.int32, "miss", 1, table.device)
-    refs = torch.empty_like(ids)
+    refs = _empty(ids.shape, ids.dtype, ids.device, _side(stream, ids.device))
     _lib.check(_lib.lib().moe_slot_lookup(
         _p(table), table.numel(), _p(ids), ids.numel(), _p(refs), _p(miss),
         _lib.stream_ptr(stream)))
@@ -169,8 +216,9 @@ def _ffn(entry, ws_entry, ws_key, pool, slot_refs, scores, x, out, out_f32, stre
     _req(x, torch.bfloat16, "x", device=pool.device)
     _req(slot_refs, torch.int32, "slot_refs", T * k, pool.device)
     _req(scores, torch.float32, "scores", T * k, pool.device)
+    side, handle = _side(stream, x.device), _lib.stream_ptr(stream)
     if out is None and out_f32 is None:
-        out = torch.empty((T, D), dtype=torch.bfloat16, device=x.device)
+        out = _empty((T, D), torch.bfloat16, x.device, side)
     if out is not None:
         _req(out, torch.bfloat16, "out", T * D, pool.device)
     if out_f32 is not None:
@@ -180,10 +228,11 @@ def _ffn(entry, ws_entry, ws_key, pool, slot_refs, scores, x, out, out_f32, stre
     need = getattr(L, ws_entry)(C.byref(g), T, k)
     if need == 0:
         raise ValueError(f"{entry}: unsupported T={T}, k={k}")
-    ws = workspace if workspace is not None else _WS.get(ws_key, need, x.device)
+    ws = workspace if workspace is not None else _WS.get(ws_key, need, x.device, handle,
+                                                         side=side)
     _lib.check(getattr(L, entry)(
         C.byref(pool.c_view()), C.byref(g), _p(slot_refs), _p(scores), _p(x),
-        T, k, _p(out), _p(out_f32), _p(ws), ws.numel(), _lib.stream_ptr(stream)))
+        T, k, _p(out), _p(out_f32), _p(ws), ws.numel(), handle))
     return out if out is not None else out_f32
 
 
@@ -228,18 +277,24 @@ def route(x: torch.Tensor, W: torch.Tensor, bias: torch.Tensor | None, mode: int
             _req(bias_next, torch.bfloat16, "bias_next", E, dev)
     if table is not None:
         _req(table, torch.int32, "table", E, dev)
-    if bufs is None:
+    side, handle = _side(stream, dev), _lib.stream_ptr(stream)
+    if bufs is None and side is None:
         bufs = RouteBuffers(T, k, k_pred, dev)
+    elif bufs is None:   # (zeroed in the stream's order, as _empty)
+        cur = torch.cuda.current_stream(dev)
+        with torch.cuda.stream(side):
+            bufs = RouteBuffers(T, k, k_pred, dev)
+        bufs.miss.record_stream(cur)   # (one allocation)
     L = _lib.lib()
     need = L.moe_route_workspace(T, E)
-    ws = workspace if workspace is not None else _WS.get("route", need, dev, zero=True)
+    ws = workspace if workspace is not None else _WS.get("route", need, dev, handle, True, side)
     _lib.check(L.moe_route(
         _p(x), T, D, _p(W), _p(bias), E, mode, int(renorm), k,
         _p(bufs.ids), _p(bufs.scores),
         _p(W_next), _p(bias_next), k_pred if W_next is not None else 0,
         _p(bufs.pred) if W_next is not None else None,
         _p(table), _p(bufs.slot_refs) if table is not None else None,
-        _p(bufs.miss), _p(ws), ws.numel(), _lib.stream_ptr(stream)))
+        _p(bufs.miss), _p(ws), ws.numel(), handle))
     return bufs
 
 

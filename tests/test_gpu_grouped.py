@@ -3,6 +3,8 @@ the grouped bf16 MFMA expert block, against the oracle on the same bytes,
 against the decode kernels on the same slot refs, and through the
 properties the grouping must not change (token order, residency, pair
 order inside a group)."""
+import threading
+
 import numpy as np
 import pytest
 import torch
@@ -522,3 +524,75 @@ def test_grouped_offset_cancels_within_four_groups(geom):
         want = step * (q * (32 * up[e, :, 0].double())).sum(1)
         t = ids == e
         assert torch.equal(y[t].double(), p[t, None].double() ** 2 * want), e
+
+
+@pytest.mark.parametrize("how", ["stream=", "current", "threads"])
+def test_calls_on_two_streams_keep_their_scratch_apart(qwen_layer, how):
+    """Routing and expert blocks of different inputs on two streams at a time,
+    with outputs and scratch of the calls' own, give what one stream gives: the
+    stream passed, made current, or each with a thread."""
+    g = qwen_layer.geom
+    runs = 8
+    xs = [[bf16_randn((T, g.d_model), seed=20260090 + 10 * s + i)
+           for i, T in enumerate([200, 9, 64, 1, 300, 17, 3, 128][:runs])] for s in range(2)]
+
+    def call(x, stream):
+        b = ops.route(x, qwen_layer.W, qwen_layer.bias, g.routing, g.norm_topk_prob, g.top_k,
+                      table=qwen_layer.table, stream=stream)
+        return b.ids, ops.ffn(qwen_layer.pool, b.slot_refs, b.scores, x, stream=stream)
+
+    want = [[call(x, None) for x in col] for col in xs]
+    torch.cuda.synchronize()
+    streams = [torch.cuda.Stream() for _ in range(2)]
+    got = [[], []]
+
+    def column(s):
+        with torch.cuda.stream(streams[s]):
+            got[s] = [call(x, None) for x in xs[s]]
+
+    if how == "threads":
+        ts = [threading.Thread(target=column, args=(s,)) for s in range(2)]
+        for t in ts:
+            t.start()
+        for t in ts:
+            t.join()
+    else:
+        for i in range(runs):
+            for s in range(2):
+                if how == "current":
+                    with torch.cuda.stream(streams[s]):
+                        got[s].append(call(xs[s][i], None))
+                else:
+                    got[s].append(call(xs[s][i], streams[s]))
+    torch.cuda.synchronize()
+    ops.check_device_error()
+    for s in range(2):
+        for (wi, wy), (gi, gy) in zip(want[s], got[s]):
+            assert torch.equal(wi, gi) and torch.equal(wy, gy), (s, wy.shape)
+
+
+def test_captured_calls_keep_scratch_of_their_own(qwen_layer):
+    """A graph captured over routing and block with default scratch, replayed with
+    the same calls made eagerly in between: every replay equals the eager result."""
+    g = qwen_layer.geom
+    x = bf16_randn((12, g.d_model), seed=20260110)
+
+    def call(v):
+        b = ops.route(v, qwen_layer.W, qwen_layer.bias, g.routing, g.norm_topk_prob, g.top_k,
+                      table=qwen_layer.table)
+        return ops.ffn(qwen_layer.pool, b.slot_refs, b.scores, v)
+
+    call(x)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        y = call(x)
+    for i in range(4):
+        x.copy_(bf16_randn(x.shape, seed=20260111 + i))
+        graph.replay()
+        torch.cuda.synchronize()
+        got = y.clone()
+        want = call(x)
+        torch.cuda.synchronize()
+        ops.check_device_error()
+        assert torch.equal(got, want), i
