@@ -29,11 +29,14 @@ HIPCC_FLAGS = [
     # no packed fp32 instructions anywhere in device code
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
     # MFMA results straight into VGPRs (no accumulator-register copies).
-    # The compiler keeps MFMA hazards itself, except against instructions
-    # written as inline asm, which it does not look into: one that writes a
-    # register which an MFMA in flight still reads gives wrong outputs.  The
-    # MFMA kernels of grouped.hip therefore decode codes with ordinary
-    # operations; their asm statements are empty.
+    # Chained MFMAs may then read an accumulator input apart from their
+    # destination, and whatever writes that input next must stay clear of them.
+    # In the built assembly no compiler-made instruction comes closer than 4
+    # issue slots to a bf16 MFMA that reads the register; instructions written
+    # as inline asm, which the compiler does not look into, come as close as 1.
+    # (To an fp32 MFMA that reads one, compiler-made ones come as close as 1.)  So
+    # the MFMA kernels decode codes with ordinary operations, their asm statements
+    # are empty, and their fp32 MFMAs start from zero.
     "-Xarch_device", "-mllvm=-amdgpu-mfma-vgpr-form=1",
     "-Wno-unused-command-line-argument",
 ]

@@ -28,14 +28,9 @@ __device__ __forceinline__ uint4 load16(const uint4 *p) {
 // store bases): as global loads.  A generic (flat) load also counts on the
 // LDS counter, so every LDS wait (each workgroup barrier among them) would
 // wait for it too.
-typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ uint4 gload16(const void *p) {
   const u32x4_t v = *(const __attribute__((address_space(1))) u32x4_t *)(p);
   return make_uint4(v.x, v.y, v.z, v.w);
-}
-__device__ __forceinline__ uint2 gload8(const void *p) {
-  const u32x2_t v = *(const __attribute__((address_space(1))) u32x2_t *)(p);
-  return make_uint2(v.x, v.y);
 }
 __device__ __forceinline__ float gload4f(const void *p) {
   return *(const __attribute__((address_space(1))) float *)(p);
@@ -79,7 +74,9 @@ __device__ __forceinline__ float dot2_bf16(uint32_t a, uint32_t b, float acc) {
                                          false);
 }
 
-// (w & M) | E in one v_bfi_b32 (E has no bits inside M).
+// (w & M) | E in one v_bfi_b32 (E has no bits inside M).  Not in MFMA kernels: the
+// compiler does not keep an inline instruction clear of the registers that an MFMA
+// in flight still reads.
 __device__ __forceinline__ uint32_t bfi_mask(uint32_t w, uint32_t M, uint32_t E) {
   uint32_t r;
   asm("v_bfi_b32 %0, %1, %2, %3" : "=v"(r) : "v"(M), "v"(w), "v"(E));

@@ -47,10 +47,11 @@ __device__ __forceinline__ f32x4_t mfma16x16x32(uint4 a, uint4 b, f32x4_t c) {
 constexpr int kTileM = 64;
 // Wide items (twice the features) from this many of them on: four rounds of the
 // 512 resident workgroups.  Below it the last round and the longest items decide,
-// and narrow items are faster (512 tokens of Qwen3 1,256 wide down items; whole
-// block with the line at 512 / 1024 / 2048 wide items: gpt-oss 29 tokens 201 / 179
-// / 166 us, 256 tokens 469 / 470 / 449, Qwen3 256 tokens 126 / 122 / 116); past it
-// the wide item's halved token-row reads win.
+// and narrow items are faster; past it the wide item's halved token-row reads win.
+// A block with the line at 1,024 / 2,048 / never: gpt-oss 29 tokens (wide from 1,024
+// on) 180 / 176 / 177 us, 60 tokens 260 / 252 / 254, 128 tokens 373 / 368 / 362;
+// Qwen3 1,024 tokens 216 / 220 / 222, 2,048 tokens 340 / 354 / 364, 4,096 tokens
+// 622 / 622 / 690.
 constexpr int kWideItems = 2048;
 
 // ---------------------------------------------------------------------------
@@ -613,8 +614,7 @@ __device__ __forceinline__ void grouped_item(
   };
   // fragment word m of 8, 4 of each code word, as pairs of bf16 128+q (one
   // v_and_or_b32 after the shift: its constants in registers, one of them scalar.
-  // Not bfi_mask(): the compiler does not see that an inline instruction writes a
-  // register that an MFMA in flight still reads)
+  // Not bfi_mask(), see there)
   uint32_t kmask = 0x000f000fu, kexp = 0x43004300u;
   asm volatile("" : "+s"(kmask));
   pin(kexp);
