@@ -592,7 +592,7 @@ __device__ __forceinline__ void grouped_item(
   // from zero, added behind the quad's folds, in the first group of the next quad:
   // there the 128 offset of the codes cancels before it is carried any further.
   float ra[M], C[N];
-  uint2 bnx = read_s(1, 0, 0);   // bias values to come
+  uint2 bcur[2];          // bias values to come
   constexpr int BZ = M <= 2 ? M : 1;
   f32x4_t bz[BZ];
 #pragma unroll
@@ -607,6 +607,7 @@ __device__ __forceinline__ void grouped_item(
     return __builtin_amdgcn_mfma_f32_16x16x4f32(ra[rb], C[n], (f32x4_t){0.f, 0.f, 0.f, 0.f}, 0, 0,
                                                 0);
   };
+  auto factor = [&](int n) { return fmaf(-128.f, pick(scur[n]), pick(bcur[n & 1])); };
   auto add_block = [&](f32x4_t &o, const f32x4_t &v) {
 #pragma unroll
     for (int e = 0; e < 4; ++e) o[e] += v[e];
@@ -688,8 +689,7 @@ __device__ __forceinline__ void grouped_item(
       const bool nxa = n == N - 1 && dec;
       const int ag = half_end ? nbuf * AG : QA ? par * AG + gi + 1 : gi + 1;
       const uint4 *an = L.a + ag * (AROWS * 8);
-      const uint2 scur_q = scur[n];
-      const uint32_t h = gi < 2 ? scur_q.x : scur_q.y;
+      const uint32_t h = gi < 2 ? scur[n].x : scur[n].y;
       S[cur] = __uint_as_float((gi & 1) ? (h & 0xffff0000u) : (h << 16));
       if (last && ng_next > 0)
 #pragma unroll
@@ -728,14 +728,15 @@ __device__ __forceinline__ void grouped_item(
         if constexpr (g0) if (bias && BZ < M) add_block(acc[rb][cb][j], bz[0]);
         __builtin_amdgcn_sched_barrier(0);
       }
-      if constexpr (g0) {   // this quad's factors
-        C[n] = fmaf(-128.f, pick(scur_q), pick(bnx));
-        if (n + 1 < N) bnx = read_s(1, q, n + 1);
-      }
-      if (last) {
-        if (ng_next > 0) bnx = read_s(1, q + 1, 0);
+      // this quad's factors, two steps behind the reads of their biases (one step
+      // of one row block is shorter than an LDS read: 8 tokens through 48 layers
+      // 2.38 ms with one step and the row sums read in a quad's last, 2.37 so)
+      if (st >= 2 && st < N + 2) C[st - 2] = factor(st - 2);
+      if constexpr (g0) {
+        bcur[st & 1] = read_s(1, q, st);
+        if (st == N - 1)
 #pragma unroll
-        for (int rb = 0; rb < M; ++rb) ra[rb] = rsl[rb * 16 * I::RSP + 4 * q];
+          for (int rb = 0; rb < M; ++rb) ra[rb] = rsl[rb * 16 * I::RSP + 4 * q];
       }
     };
     // (two loops, each small enough to be unrolled)
@@ -759,6 +760,10 @@ __device__ __forceinline__ void grouped_item(
     quad(q, q & 1, groups(q), groups(q + 1), groups(q + R), groups(q + 1 + R), q == 0);
   }
   {   // the last step's fold and the last quad's bias term
+    if (NGL == 1) {   // (too short for its last two factors)
+      C[N - 2] = factor(N - 2);
+      C[N - 1] = factor(N - 1);
+    }
     constexpr int last = (NGL * N - 1) & 1, lc = (N - 1) / NPROJ, lj = (N - 1) % NPROJ;
 #pragma unroll
     for (int rb = 0; rb < M; ++rb) {
