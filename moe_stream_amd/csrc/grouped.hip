@@ -258,8 +258,9 @@ __global__ __launch_bounds__(1024) void group_prep_kernel(
 //
 // Measured (whole block against the kernels before these: 64-row tiles with codes
 // and rows staged a quad at a time behind two barriers, narrow items only, cold
-// weights; results bit for bit the same): Qwen3 4,096 tokens 694 -> 587 us, 512
-// tokens 147 -> 145, gpt-oss 700 tokens 750 -> 605, 29 tokens 212 -> 178.
+// weights; results bit for bit the same): Qwen3 4,096 tokens 704 -> 596 us, 512
+// tokens 145 -> 142, gpt-oss 700 tokens 743 -> 608, 29 tokens 211 -> 173; 8 and 16 Qwen3
+// tokens through 48 layers 2.34 -> 2.37 and 2.73 -> 2.79 ms.
 //
 // What sets the shape: per group a wave's M x N blocks (N = CB * NPROJ) take
 // 32 M N matrix-core cycles (8 M N more for the bias term), 64 M LDS cycles (a

@@ -191,8 +191,8 @@ def ffn_grouped(pool, slot_refs: torch.Tensor, scores: torch.Tensor,
 # the decode kernels (which group the pairs by slot from 2 tokens on and give
 # results bit-identical to one call per token).  Per step of the 48-layer
 # Qwen3 stack on one MI355X (HIP graph of router + expert block per layer):
-# 4 tokens 2.03 ms (decode kernels) vs 2.02 ms (MFMA block), 8 tokens 2.81
-# vs 2.37 ms, 16 tokens 4.35 vs 2.74 ms.
+# 4 tokens 2.05 ms (decode kernels) vs 1.97 ms (MFMA block), 8 tokens 2.80
+# vs 2.38 ms, 16 tokens 4.33 vs 2.79 ms.
 GROUPED_MIN_TOKENS = 4
 
 
